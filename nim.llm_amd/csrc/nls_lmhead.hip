@@ -29,6 +29,7 @@
 #include <algorithm>
 
 #include "nls_internal.h"
+#include "nls_lmhead.h"
 
 namespace nls {
 namespace {
@@ -38,19 +39,9 @@ constexpr int kLmNBC = 4;    // activation rows per pass over a row group
 
 // ---------------------------------------------------------------- loads
 
-__device__ __forceinline__ uint32_t ld_u16(const uint8_t* p) {
-  uint16_t v;
-  __builtin_memcpy(&v, p, 2);
-  return v;
-}
 __device__ __forceinline__ uint2 ld_8(const void* p) {
   uint2 v;
   __builtin_memcpy(&v, p, 8);
-  return v;
-}
-__device__ __forceinline__ uint4 ld_16(const void* p) {
-  uint4 v;
-  __builtin_memcpy(&v, p, 16);
   return v;
 }
 // 4-byte aligned words covering NW * 4 bytes at a 2-byte aligned address,
@@ -76,13 +67,6 @@ __device__ __forceinline__ void ld_words_a(const uint8_t* p, uint32_t (&out)[NW]
   for (int k = 0; k < NW; ++k) out[k] = __builtin_amdgcn_alignbit(w[k + 1], w[k], sh);
 }
 
-// IEEE half to float: exact for every finite half (subnormals included).
-__device__ __forceinline__ float half_f(uint32_t bits) {
-  _Float16 h;
-  const uint16_t b = (uint16_t)bits;
-  __builtin_memcpy(&h, &b, 2);
-  return (float)h;
-}
 __device__ __forceinline__ int dot4(uint32_t a, uint32_t b, int c) {
   return __builtin_amdgcn_sdot4((int)a, (int)b, c, false);
 }
@@ -175,7 +159,7 @@ struct Fmt<14> {
     w.ql1 = ld_8(blk + 64 * h + 32 + l0);
     w.qh = ld_8(blk + 128 + 32 * h + l0);
     w.sc = ld_8(blk + 192 + 8 * h);
-    w.d = ld_u16(blk + 208);
+    w.d = lm_ld_u16(blk + 208);
     return w;
   }
   static constexpr bool HAS_MIN = false;
@@ -214,7 +198,7 @@ struct Fmt<14> {
   }
   // acc += a.d * d * sumi  (quant.nim:759)
   __device__ static float term(const Wt& w, int sumi, int, float ad) {
-    return __fmul_rn(__fmul_rn(ad, half_f(w.d)), (float)sumi);
+    return __fmul_rn(__fmul_rn(ad, lm_half_f(w.d)), (float)sumi);
   }
 };
 
@@ -236,9 +220,9 @@ struct FmtK45 {
   __device__ static Wt load_w(const uint8_t* blk, int p) {
     const int j = p >> 1, l0 = 16 * (p & 1);
     Wt w;
-    w.hd = ld_16(blk);
-    w.qs = ld_16(blk + (FIVE ? 48 : 16) + 32 * j + l0);
-    if (FIVE) w.qh = ld_16(blk + 16 + l0);
+    w.hd = lm_ld_16(blk);
+    w.qs = lm_ld_16(blk + (FIVE ? 48 : 16) + 32 * j + l0);
+    if (FIVE) w.qh = lm_ld_16(blk + 16 + l0);
     return w;
   }
   static constexpr bool HAS_MIN = true;
@@ -292,7 +276,7 @@ struct FmtK45 {
   }
   // acc += a.d * (d * sumi - dmin * summ)  (quant.nim:694, :728)
   __device__ static float term(const Wt& w, int sumi, int summ, float ad) {
-    const float d = half_f(w.hd.x & 0xFFFF), dmin = half_f(w.hd.x >> 16);
+    const float d = lm_half_f(w.hd.x & 0xFFFF), dmin = lm_half_f(w.hd.x >> 16);
     return __fmul_rn(ad, __fsub_rn(__fmul_rn(d, (float)sumi), __fmul_rn(dmin, (float)summ)));
   }
 };
@@ -314,7 +298,7 @@ struct Fmt<8> {
   };
   __device__ static Wt load_w(const uint8_t* blk, int) {
     Wt w;
-    w.d = ld_u16(blk);
+    w.d = lm_ld_u16(blk);
     uint32_t q[8];
     ld_words_a<8>(blk + 2, q);
     w.q0 = make_uint4(q[0], q[1], q[2], q[3]);
@@ -340,7 +324,7 @@ struct Fmt<8> {
   }
   // acc += rdHalf(w, o) * a.d * s  (quant.nim:771)
   __device__ static float term(const Wt& w, int sumi, int, float ad) {
-    return __fmul_rn(__fmul_rn(half_f(w.d), ad), (float)sumi);
+    return __fmul_rn(__fmul_rn(lm_half_f(w.d), ad), (float)sumi);
   }
 };
 
@@ -358,7 +342,7 @@ struct Fmt<2> {
   };
   __device__ static Wt load_w(const uint8_t* blk, int) {
     Wt w;
-    w.d = ld_u16(blk);
+    w.d = lm_ld_u16(blk);
     uint32_t q[4];
     ld_words_a<4>(blk + 2, q);
     w.q = make_uint4(q[0], q[1], q[2], q[3]);
@@ -390,7 +374,7 @@ struct Fmt<2> {
     summ = 0;
   }
   __device__ static float term(const Wt& w, int sumi, int, float ad) {
-    return __fmul_rn(__fmul_rn(half_f(w.d), ad), (float)sumi);
+    return __fmul_rn(__fmul_rn(lm_half_f(w.d), ad), (float)sumi);
   }
 };
 
@@ -642,11 +626,11 @@ __device__ __forceinline__ float deq1<0>(const uint8_t* rp, int64_t e) {  // F32
 }
 template <>
 __device__ __forceinline__ float deq1<1>(const uint8_t* rp, int64_t e) {  // F16
-  return half_f(ld_u16(rp + 2 * e));
+  return lm_half_f(lm_ld_u16(rp + 2 * e));
 }
 template <>
 __device__ __forceinline__ float deq1<30>(const uint8_t* rp, int64_t e) {  // BF16
-  return __uint_as_float(ld_u16(rp + 2 * e) << 16);
+  return __uint_as_float(lm_ld_u16(rp + 2 * e) << 16);
 }
 template <>
 __device__ __forceinline__ float deq1<2>(const uint8_t* rp, int64_t e) {  // Q4_0 :167-172
@@ -654,7 +638,7 @@ __device__ __forceinline__ float deq1<2>(const uint8_t* rp, int64_t e) {  // Q4_
   const int i = (int)(e & 31);
   const uint32_t q = b[2 + (i & 15)];
   const int v = (int)(i < 16 ? (q & 0xF) : (q >> 4)) - 8;
-  return __fmul_rn((float)v, half_f(ld_u16(b)));
+  return __fmul_rn((float)v, lm_half_f(lm_ld_u16(b)));
 }
 template <>
 __device__ __forceinline__ float deq1<3>(const uint8_t* rp, int64_t e) {  // Q4_1 :173-179
@@ -662,7 +646,7 @@ __device__ __forceinline__ float deq1<3>(const uint8_t* rp, int64_t e) {  // Q4_
   const int i = (int)(e & 31);
   const uint32_t q = b[4 + (i & 15)];
   const uint32_t v = i < 16 ? (q & 0xF) : (q >> 4);
-  return __fadd_rn(__fmul_rn((float)v, half_f(ld_u16(b))), half_f(ld_u16(b + 2)));
+  return __fadd_rn(__fmul_rn((float)v, lm_half_f(lm_ld_u16(b))), lm_half_f(lm_ld_u16(b + 2)));
 }
 template <>
 __device__ __forceinline__ float deq1<6>(const uint8_t* rp, int64_t e) {  // Q5_0 :180-188
@@ -672,7 +656,7 @@ __device__ __forceinline__ float deq1<6>(const uint8_t* rp, int64_t e) {  // Q5_
   __builtin_memcpy(&qh, b + 2, 4);
   const uint32_t q = b[6 + j];
   const uint32_t v = i < 16 ? ((q & 0xF) | (((qh >> j) << 4) & 0x10)) : ((q >> 4) | ((qh >> (j + 12)) & 0x10));
-  return __fmul_rn((float)((int)v - 16), half_f(ld_u16(b)));
+  return __fmul_rn((float)((int)v - 16), lm_half_f(lm_ld_u16(b)));
 }
 template <>
 __device__ __forceinline__ float deq1<7>(const uint8_t* rp, int64_t e) {  // Q5_1 :189-198
@@ -682,20 +666,20 @@ __device__ __forceinline__ float deq1<7>(const uint8_t* rp, int64_t e) {  // Q5_
   __builtin_memcpy(&qh, b + 4, 4);
   const uint32_t q = b[8 + j];
   const uint32_t v = i < 16 ? ((q & 0xF) | (((qh >> j) << 4) & 0x10)) : ((q >> 4) | ((qh >> (j + 12)) & 0x10));
-  return __fadd_rn(__fmul_rn((float)v, half_f(ld_u16(b))), half_f(ld_u16(b + 2)));
+  return __fadd_rn(__fmul_rn((float)v, lm_half_f(lm_ld_u16(b))), lm_half_f(lm_ld_u16(b + 2)));
 }
 template <>
 __device__ __forceinline__ float deq1<8>(const uint8_t* rp, int64_t e) {  // Q8_0 :199-202
   const uint8_t* b = rp + 34 * (e >> 5);
-  return __fmul_rn((float)(int8_t)b[2 + (e & 31)], half_f(ld_u16(b)));
+  return __fmul_rn((float)(int8_t)b[2 + (e & 31)], lm_half_f(lm_ld_u16(b)));
 }
 template <>
 __device__ __forceinline__ float deq1<10>(const uint8_t* rp, int64_t e) {  // Q2_K :207-228
   const uint8_t* b = rp + 84 * (e >> 8);
   const int i = (int)(e & 255), n = i >> 7, j = (i >> 5) & 3, l = i & 31;
   const uint32_t sc = b[i >> 4];
-  const float dl = __fmul_rn(half_f(ld_u16(b + 80)), (float)(sc & 0xF));
-  const float ml = __fmul_rn(half_f(ld_u16(b + 82)), (float)(sc >> 4));
+  const float dl = __fmul_rn(lm_half_f(lm_ld_u16(b + 80)), (float)(sc & 0xF));
+  const float ml = __fmul_rn(lm_half_f(lm_ld_u16(b + 82)), (float)(sc >> 4));
   const uint32_t q = (b[16 + 32 * n + l] >> (2 * j)) & 3;
   return __fsub_rn(__fmul_rn(dl, (float)q), ml);
 }
@@ -708,7 +692,7 @@ __device__ __forceinline__ float deq1<11>(const uint8_t* rp, int64_t e) {  // Q3
   const uint32_t lo = s < 8 ? (b[96 + s] & 0xF) : (b[96 + s - 8] >> 4);
   const uint32_t hi = (b[104 + (s & 3)] >> (2 * (s >> 2))) & 3;
   const int scale = (int)(lo | (hi << 4));
-  const float dl = __fmul_rn(half_f(ld_u16(b + 108)), (float)(scale - 32));
+  const float dl = __fmul_rn(lm_half_f(lm_ld_u16(b + 108)), (float)(scale - 32));
   const int hv = (b[l] & (1u << (4 * n + j))) != 0 ? 0 : 4;
   const int q = (int)((b[32 + 32 * n + l] >> (2 * j)) & 3) - hv;
   return __fmul_rn(dl, (float)q);
@@ -718,10 +702,10 @@ __device__ __forceinline__ float deq1_k45(const uint8_t* rp, int64_t e) {  // :2
   const uint8_t* b = rp + (FIVE ? 176 : 144) * (e >> 8);
   const int i = (int)(e & 255), jj = i >> 6, hi = (i >> 5) & 1, l = i & 31;
   int sc, mn;
-  const uint4 hd = ld_16(b);
+  const uint4 hd = lm_ld_16(b);
   FmtK45<FIVE>::scale_min(hd, 2 * jj + hi, sc, mn);
-  const float d1 = __fmul_rn(half_f(hd.x & 0xFFFF), (float)sc);
-  const float m1 = __fmul_rn(half_f(hd.x >> 16), (float)mn);
+  const float d1 = __fmul_rn(lm_half_f(hd.x & 0xFFFF), (float)sc);
+  const float m1 = __fmul_rn(lm_half_f(hd.x >> 16), (float)mn);
   const uint32_t byte = b[(FIVE ? 48 : 16) + 32 * jj + l];
   int q = (int)(hi ? (byte >> 4) : (byte & 0xF));
   if (FIVE) q += ((b[16 + l] >> (2 * jj + hi)) & 1) ? 16 : 0;
@@ -744,7 +728,7 @@ __device__ __forceinline__ float deq1<14>(const uint8_t* rp, int64_t e) {  // Q6
   const uint32_t hb = (b[128 + 32 * n + l] >> (2 * m)) & 3;
   const int q = (int)(nib | (hb << 4)) - 32;
   const int sc = (int8_t)b[192 + 8 * n + (l >> 4) + 2 * m];
-  return __fmul_rn(__fmul_rn(half_f(ld_u16(b + 208)), (float)sc), (float)q);
+  return __fmul_rn(__fmul_rn(lm_half_f(lm_ld_u16(b + 208)), (float)sc), (float)q);
 }
 template <>
 __device__ __forceinline__ float deq1<15>(const uint8_t* rp, int64_t e) {  // Q8_K :321-324
@@ -768,18 +752,18 @@ template <int T>
 __device__ __forceinline__ void deq8(const uint8_t* __restrict__ rp, int64_t e0, int64_t cols, float (&w)[8]) {
   if (e0 + 8 <= cols) {
     if constexpr (T == 0) {  // F32: two 16-byte loads
-      const uint4 a = ld_16(rp + 4 * e0), b = ld_16(rp + 4 * e0 + 16);
+      const uint4 a = lm_ld_16(rp + 4 * e0), b = lm_ld_16(rp + 4 * e0 + 16);
       const uint32_t u[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
       for (int j = 0; j < 8; ++j) w[j] = __uint_as_float(u[j]);
     } else if constexpr (T == 1 || T == 30) {  // F16, BF16: one 16-byte load
-      const uint4 a = ld_16(rp + 2 * e0);
+      const uint4 a = lm_ld_16(rp + 2 * e0);
       const uint32_t u[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         if constexpr (T == 1) {
-          w[2 * j] = half_f(u[j] & 0xFFFF);
-          w[2 * j + 1] = half_f(u[j] >> 16);
+          w[2 * j] = lm_half_f(u[j] & 0xFFFF);
+          w[2 * j + 1] = lm_half_f(u[j] >> 16);
         } else {
           w[2 * j] = __uint_as_float(u[j] << 16);
           w[2 * j + 1] = __uint_as_float(u[j] & 0xFFFF0000u);
@@ -805,10 +789,10 @@ __device__ __forceinline__ Raw8 raw8(const uint8_t* __restrict__ rp, int64_t e0,
   Raw8 r{make_uint4(0u, 0u, 0u, 0u), make_uint4(0u, 0u, 0u, 0u)};
   if (e0 + 8 <= cols) {
     if constexpr (T == 0) {
-      r.a = ld_16(rp + 4 * e0);
-      r.b = ld_16(rp + 4 * e0 + 16);
+      r.a = lm_ld_16(rp + 4 * e0);
+      r.b = lm_ld_16(rp + 4 * e0 + 16);
     } else {
-      r.a = ld_16(rp + 2 * e0);
+      r.a = lm_ld_16(rp + 2 * e0);
     }
   }
   return r;
@@ -824,8 +808,8 @@ __device__ __forceinline__ void cvt8(const Raw8& r, float (&w)[8]) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       if constexpr (T == 1) {
-        w[2 * j] = half_f(u[j] & 0xFFFF);
-        w[2 * j + 1] = half_f(u[j] >> 16);
+        w[2 * j] = lm_half_f(u[j] & 0xFFFF);
+        w[2 * j + 1] = lm_half_f(u[j] >> 16);
       } else {
         w[2 * j] = __uint_as_float(u[j] << 16);
         w[2 * j + 1] = __uint_as_float(u[j] & 0xFFFF0000u);
@@ -1016,6 +1000,7 @@ hipError_t launch_int(const LmHeadCall& c, hipStream_t s) {
   hipLaunchKernelGGL(quant_act_kernel<F::BL>, dim3((unsigned)qgrid), dim3(kLmNT), 0, s, c.x, n, c.act_qs, c.act_d);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
+  if (lm_batch_serves(T, c.rows, c.nb)) return launch_lm_batch(c, s);
   IntArgs a;
   a.w = static_cast<const uint8_t*>(c.w);
   a.rows = c.rows;

@@ -207,3 +207,43 @@ def test_lm_head_random_cases(pkg, i):
     t, rows, cols, nb, exact, rank = _drawn_lm_case(i)
     print(f"lm_head sweep {i}: type={t} rows={rows} cols={cols} nb={nb} exact={exact} lora={rank}", flush=True)
     run_case(pkg, t, rows, cols, nb, exact=exact, lora_rank=rank, seed=900 + i)
+
+
+def _extreme_weights(t, rows, cols, rng):
+    """Random K-format rows of which every third block has its scales, mins and
+    levels at their largest (the widest integer sums the formats hold)."""
+    raw = rand_weights(t, rows, cols, rng)
+    blocks = raw.reshape(rows, -1, O.type_size(t))
+    heads = {O.GGML["Q4_K"]: (4, 16), O.GGML["Q5_K"]: (4, 16), O.GGML["Q6_K"]: (192, 208)}[t]
+    for i in range(0, blocks.shape[1], 3):
+        keep = blocks[:, i].copy()
+        blocks[:, i] = 0xFF if i % 2 else 0x00
+        for off in HALF_FIELDS[t]:
+            blocks[:, i, off:off + 2] = keep[:, off:off + 2]
+        blocks[:, i, heads[0]:heads[1]] = 0x80 if t == O.GGML["Q6_K"] else 0xFF
+    return raw
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["Q4_K", "Q5_K", "Q6_K"])
+def test_batched_states_parity(pkg, name):
+    """More than four hidden states (the matrix-core path): row counts around
+    a wave's 32 and a workgroup's 128 rows, state counts around one tile (32)
+    and one workgroup's four (128), one to nine blocks per row, and the
+    integer sums at their widest (activations all at +-127, extreme scales):
+    every logit bit for bit (integer sums are exact, the fp32 terms ordered)."""
+    import torch
+
+    t = TYPES[name]
+    for rows, nb, blocks in [(1, 5, 1), (31, 32, 2), (33, 33, 1), (127, 6, 9), (129, 31, 3), (300, 64, 2), (65, 97, 2),
+                             (128, 128, 1), (257, 129, 2), (40, 255, 2), (1000, 24, 8), (5, 300, 1)]:
+        print(f"lm_head batch {name} rows={rows} cols={256 * blocks} nb={nb}", flush=True)
+        run_case(pkg, t, rows, 256 * blocks, nb, seed=rows + nb)
+    rng = np.random.default_rng(4)
+    rows, cols, nb = 96, 768, 40
+    w = _extreme_weights(t, rows, cols, rng)
+    x = np.where(rng.random((nb, cols)) < 0.1, -1.0, 1.0).astype(F32)
+    x[::2] = 1.0
+    want = O.matmul(t, w, rows, cols, x)
+    got = pkg.lm_head(torch.from_numpy(w).cuda(), t, rows, cols, torch.from_numpy(x).cuda()).cpu().numpy()
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
