@@ -29,9 +29,14 @@
 // across lanes, so the block scales are one value per lane and the stores are
 // contiguous.
 //
-// Bound: at few states the weights' HBM traffic, at many the matrix unit (two
-// planes: 32 cycles per 32 x 32 x 32 step) beside about 6 VALU instructions
-// per term.
+// Bound: at few states the weights' HBM traffic and the making of the planes
+// (about 2 VALU instructions per 4 weights and plane for Q4_K, 7 for Q6_K), at
+// many the matrix unit (two planes, 32 cycles per 32 x 32 x 32 step: 57 us of
+// the 195 at 255 states) and the 5 to 7 VALU instructions per term (89 us),
+// which two waves per SIMD overlap only in part.  128256 x 2048, before (one
+// dot-product instruction per four products, weights re-read per four states)
+// and now: Q4_K, 255 states 4009 -> 207 us; Q6_K, 24 states 571 -> 79 us,
+// 5 states 174 -> 79 us; Q6_K 32000 x 4096, 3 states 99 -> 55 us.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -268,12 +273,17 @@ __global__ __launch_bounds__(kBNT, 2) void lm_batch_kernel(BatchArgs a) {
   for (int t = 0; t < TILES; ++t) acc[t] = v16f{};
   for (int ib = 0; ib < a.nblk; ++ib) {
     const int buf = ib & 1;
+    const bool more = ib + 1 < a.nblk;
+    const int nx = more ? ib + 1 : ib;  // (the last block is requested twice; nothing reads the second)
+    // loads are waited for in order: the first tile's next activations (L2)
+    // go out before the next weights (HBM), both as early as registers allow
+    v4i nxt[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) nxt[u] = *reinterpret_cast<const v4i*>(src(0, nx, u));
     v4i L[8], H[8];
     v8h mins{};
     float d, dmin = 0.0f;
     raw.planes(h, L, H, mins, d, dmin);
-    const bool more = ib + 1 < a.nblk;
-    const int nx = more ? ib + 1 : ib;  // (the last block is requested twice; nothing reads the second)
     raw.load(wrow + (int64_t)nx * R::TS, h);
     // block ib's activations are in; every wave is past block ib - 1, whose
     // buffer takes block ib + 1's
@@ -281,9 +291,10 @@ __global__ __launch_bounds__(kBNT, 2) void lm_batch_kernel(BatchArgs a) {
     put_ad(buf ^ 1, nx);
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
-      v4i nxt[2];
+      if (t > 0) {
 #pragma unroll
-      for (int u = 0; u < 2; ++u) nxt[u] = *reinterpret_cast<const v4i*>(src(t, nx, u));
+        for (int u = 0; u < 2; ++u) nxt[u] = *reinterpret_cast<const v4i*>(src(t, nx, u));
+      }
       v16i sl{}, sh{};
 #pragma unroll
       for (int s = 0; s < 8; ++s) {
@@ -333,6 +344,8 @@ hipError_t launch_type(const LmHeadCall& c, hipStream_t s) {
               0, (int)((c.rows + kBRows - 1) / kBRows), c.y};
   const int tiles = (c.nb + 31) / 32;
   a.groups = (tiles + kBTiles - 1) / kBTiles;
+  // (the grid's index is 32 bits; a matrix past this does not fit the memory)
+  if ((c.rows + kBRows - 1) / kBRows > (int64_t{1} << 29) / a.groups) return hipErrorInvalidConfiguration;
   const int per = (tiles + a.groups - 1) / a.groups;
   switch (per) {
     case 1: launch<T, 1>(a, s); break;
@@ -344,11 +357,6 @@ hipError_t launch_type(const LmHeadCall& c, hipStream_t s) {
 }
 
 }  // namespace
-
-bool lm_batch_serves(int type, int64_t rows, int nb) {
-  const int64_t groups = ((int64_t)nb + 127) / 128, tiles = (rows + kBRows - 1) / kBRows;
-  return (type == 12 || type == 13 || type == 14) && nb > 4 && tiles <= (int64_t{1} << 29) / groups;
-}
 
 hipError_t launch_lm_batch(const LmHeadCall& c, hipStream_t s) {
   switch (c.type) {

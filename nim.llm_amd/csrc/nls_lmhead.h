@@ -25,9 +25,8 @@ __device__ __forceinline__ float lm_half_f(uint32_t bits) {
   return (float)h;
 }
 
-// nls_lmbatch.hip: the int8 path for more than four hidden states on the
-// matrix cores, after the activations are quantised into the workspace.
-bool lm_batch_serves(int type, int64_t rows, int nb);
+// nls_lmbatch.hip: the K formats' int8 path on the matrix cores, after the
+// activations are quantised into the workspace.
 hipError_t launch_lm_batch(const LmHeadCall& c, hipStream_t s);
 
 }  // namespace nls

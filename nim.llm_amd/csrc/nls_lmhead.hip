@@ -441,14 +441,16 @@ struct IntArgs {
   float* y;
 };
 
-// One wave per group of `rw` rows.  For each row the wave's lanes form the
-// integer partials of their slices (64 slices = 2048 weights per pass), the
-// 8 lanes of a block add theirs, and the block's last lane writes the block's
-// fp32 term to LDS.  Then one lane per row adds its row's terms in block
-// order.  Up to kLmNBC activation rows share each load of a weight slice.
+// The 32-weight formats past lm_int1_kernel's reach (Q4_0 with more than four
+// hidden states, long rows).  One wave per group of `rw` rows.  For each row
+// the wave's lanes form the integer sums of their blocks (64 blocks = 2048
+// weights per pass) and write the blocks' fp32 terms to LDS.  Then one lane
+// per row adds its row's terms in block order.  Up to kLmNBC activation rows
+// share each load of a block.
 template <int T>
 __global__ __launch_bounds__(kLmNT) void lm_int_kernel(IntArgs a) {
   using F = Fmt<T>;
+  static_assert(F::LPB == 1, "one lane per block");
   extern __shared__ float s_term[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int64_t row0 = ((int64_t)blockIdx.x * (kLmNT / 64) + wave) * a.rw;
@@ -456,30 +458,20 @@ __global__ __launch_bounds__(kLmNT) void lm_int_kernel(IntArgs a) {
   const int nrow = (int)min<int64_t>(a.rw, a.rows - row0);
   const int nbc_max = min(a.nb, kLmNBC);
   float* term = s_term + (size_t)wave * nbc_max * a.rw * a.nblk;
-  const int S = (int)(a.cols / 32);  // 32-weight slices per row
   for (int b0 = 0; b0 < a.nb; b0 += kLmNBC) {
     const int nbc = min(kLmNBC, a.nb - b0);
     for (int rr = 0; rr < nrow; ++rr) {
       const uint8_t* rp = a.w + (row0 + rr) * a.row_bytes;
       for (int pass = 0; pass < a.passes; ++pass) {
-        const int s = pass * 64 + lane;
-        const bool on = s < S;
-        const int ib = s / F::LPB, p = s % F::LPB;
-        typename F::Wt w{};
-        if (on) w = F::load_w(rp + (int64_t)ib * F::TS, p);
+        const int ib = pass * 64 + lane;
+        if (ib >= a.nblk) continue;
+        const typename F::Wt w = F::load_w(rp + (int64_t)ib * F::TS, 0);
         for (int bb = 0; bb < nbc; ++bb) {
           const int64_t brow = b0 + bb;
-          int si = 0, sm = 0;
-          if (on) {
-            const typename F::Act act = load_act<T>(a.aqs + brow * a.cols + (int64_t)ib * F::BL, p);
-            F::partial(w, act, p, si, sm);
-          }
-          if (F::LPB == 8) {
-            si = group8_sum(si);
-            if (F::HAS_MIN) sm = group8_sum(sm);
-          }
-          if (on && p == F::LPB - 1)
-            term[(bb * a.rw + rr) * a.nblk + ib] = F::term(w, si, sm, a.ad[brow * a.nblk + ib]);
+          const typename F::Act act = load_act<T>(a.aqs + brow * a.cols + (int64_t)ib * F::BL, 0);
+          int si, sm;
+          F::partial(w, act, 0, si, sm);
+          term[(bb * a.rw + rr) * a.nblk + ib] = F::term(w, si, sm, a.ad[brow * a.nblk + ib]);
         }
       }
     }
@@ -982,25 +974,7 @@ hipError_t launch_int1(const LmHeadCall& c, int nblk, hipStream_t s) {
 }
 
 template <int T>
-hipError_t launch_int(const LmHeadCall& c, hipStream_t s) {
-  using F = Fmt<T>;
-  const int nblk = (int)(c.cols / F::BL);
-  const int passes = (int)((c.cols / 32 + 63) / 64);
-  // up to four hidden states with each weight slice loaded once for all;
-  // activation slices held in registers for nb x passes <= 4
-  if (c.nb == 1 && passes <= 4) {
-    if (passes == 1) return launch_int1<T, 1, 1>(c, nblk, s);
-    if (passes == 2) return launch_int1<T, 2, 1>(c, nblk, s);
-    return launch_int1<T, 4, 1>(c, nblk, s);
-  }
-  if (c.nb == 2 && passes <= 2) return passes == 1 ? launch_int1<T, 1, 2>(c, nblk, s) : launch_int1<T, 2, 2>(c, nblk, s);
-  if (c.nb <= 4 && passes == 1) return launch_int1<T, 1, 4>(c, nblk, s);
-  const int64_t n = (int64_t)c.nb * c.cols;
-  const int64_t qgrid = (n / 4 + kLmNT - 1) / kLmNT;
-  hipLaunchKernelGGL(quant_act_kernel<F::BL>, dim3((unsigned)qgrid), dim3(kLmNT), 0, s, c.x, n, c.act_qs, c.act_d);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  if (lm_batch_serves(T, c.rows, c.nb)) return launch_lm_batch(c, s);
+hipError_t launch_int32(const LmHeadCall& c, int nblk, int passes, hipStream_t s) {
   IntArgs a;
   a.w = static_cast<const uint8_t*>(c.w);
   a.rows = c.rows;
@@ -1021,6 +995,29 @@ hipError_t launch_int(const LmHeadCall& c, hipStream_t s) {
   const int64_t grid = (c.rows + (int64_t)rw * (kLmNT / 64) - 1) / ((int64_t)rw * (kLmNT / 64));
   hipLaunchKernelGGL(lm_int_kernel<T>, dim3((unsigned)grid), dim3(kLmNT), lds, s, a);
   return hipGetLastError();
+}
+
+template <int T>
+hipError_t launch_int(const LmHeadCall& c, hipStream_t s) {
+  using F = Fmt<T>;
+  const int nblk = (int)(c.cols / F::BL);
+  const int passes = (int)((c.cols / 32 + 63) / 64);
+  // up to four hidden states with each weight slice loaded once for all;
+  // activation slices held in registers for nb x passes <= 4
+  if (c.nb == 1 && passes <= 4) {
+    if (passes == 1) return launch_int1<T, 1, 1>(c, nblk, s);
+    if (passes == 2) return launch_int1<T, 2, 1>(c, nblk, s);
+    return launch_int1<T, 4, 1>(c, nblk, s);
+  }
+  if (c.nb == 2 && passes <= 2) return passes == 1 ? launch_int1<T, 1, 2>(c, nblk, s) : launch_int1<T, 2, 2>(c, nblk, s);
+  if (c.nb <= 4 && passes == 1) return launch_int1<T, 1, 4>(c, nblk, s);
+  const int64_t n = (int64_t)c.nb * c.cols;
+  const int64_t qgrid = (n / 4 + kLmNT - 1) / kLmNT;
+  hipLaunchKernelGGL(quant_act_kernel<F::BL>, dim3((unsigned)qgrid), dim3(kLmNT), 0, s, c.x, n, c.act_qs, c.act_d);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  if constexpr (F::LPB == 8) return launch_lm_batch(c, s);
+  else return launch_int32<T>(c, nblk, passes, s);
 }
 
 template <int T>

@@ -239,6 +239,10 @@ def test_batched_states_parity(pkg, name):
                              (128, 128, 1), (257, 129, 2), (40, 255, 2), (1000, 24, 8), (5, 300, 1)]:
         print(f"lm_head batch {name} rows={rows} cols={256 * blocks} nb={nb}", flush=True)
         run_case(pkg, t, rows, 256 * blocks, nb, seed=rows + nb)
+    # few states of rows past what one lane's registers hold
+    for rows, nb, blocks in [(70, 1, 33), (33, 2, 17), (130, 3, 9), (64, 4, 16)]:
+        print(f"lm_head long rows {name} rows={rows} cols={256 * blocks} nb={nb}", flush=True)
+        run_case(pkg, t, rows, 256 * blocks, nb, seed=rows + nb)
     rng = np.random.default_rng(4)
     rows, cols, nb = 96, 768, 40
     w = _extreme_weights(t, rows, cols, rng)
