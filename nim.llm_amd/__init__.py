@@ -36,6 +36,7 @@ EXPORTED = (
     "nls_sample_host_noalloc",
     "nls_synchronize", "nls_rng_uniforms", "nls_get_rng_state", "nls_set_rng_state",
     "nls_top_tokens", "nls_row_nll", "nls_softmax_rows", "nls_log_prob", "nls_expf_device",
+    "nls_rows_workspace", "nls_top_tokens_ws", "nls_row_nll_ws", "nls_softmax_rows_ws", "nls_log_prob_ws",
     "nls_profile_next",
     "nls_profile_next_generic", "nls_get_plan", "nls_status_string", "nls_last_error",
     "nls_lm_head_workspace", "nls_lm_head", "nls_lm_head_row_bytes", "nls_argmax",
@@ -132,6 +133,13 @@ def lib():
         L.nls_row_nll.argtypes = [vp, ctypes.c_int32, ctypes.c_int64, vp, vp, vp]
         L.nls_softmax_rows.argtypes = [vp, ctypes.c_int32, ctypes.c_int64, vp, vp]
         L.nls_log_prob.argtypes = [vp, ctypes.c_int32, ctypes.c_int64, vp, vp, vp, vp]
+        L.nls_rows_workspace.argtypes = [ctypes.c_int32, ctypes.c_int32, ctypes.c_int64, ctypes.c_int32]
+        L.nls_rows_workspace.restype = ctypes.c_size_t
+        ws = [vp, ctypes.c_size_t, vp]  # the workspace, its bytes, the stream
+        L.nls_top_tokens_ws.argtypes = L.nls_top_tokens.argtypes[:-1] + ws
+        L.nls_row_nll_ws.argtypes = L.nls_row_nll.argtypes[:-1] + ws
+        L.nls_softmax_rows_ws.argtypes = L.nls_softmax_rows.argtypes[:-1] + ws
+        L.nls_log_prob_ws.argtypes = L.nls_log_prob.argtypes[:-1] + ws
         L.nls_expf_device.argtypes = [vp, vp, ctypes.c_int64, vp]
         L.nls_profile_next.argtypes = [vp, vp, vp]
         L.nls_profile_next_generic.argtypes = [vp, vp, vp]
@@ -421,6 +429,19 @@ def newSampler(p: Optional[SamplerParams] = None, vocab: int = 0) -> Sampler:
 TOP_TOKENS_MAX = 2048  # largest number of entries per row nls_top_tokens returns
 
 
+# nls_rows_workspace's calls
+_ROWS_SOFTMAX, _ROWS_LOG_PROB, _ROWS_TOP_TOKENS, _ROWS_NLL = range(4)
+
+
+def _rows_work(op: int, x, n: int = 0):
+    """The workspace of a call over the rows of x (None where it wants none),
+    from torch's allocator on the current stream, and its bytes."""
+    import torch
+
+    need = int(lib().nls_rows_workspace(op, x.shape[0], x.shape[1], n))
+    return (torch.empty(need, dtype=torch.uint8, device=x.device) if need else None), need
+
+
 def top_tokens_device(logits, n: int = 5):
     """topTokens (sampler.nim:123-130) for a [rows, V] float32 device tensor:
     returns int32 ids and float32 probabilities, both [rows, min(n, V)], in the
@@ -434,9 +455,10 @@ def top_tokens_device(logits, n: int = 5):
     ids = torch.empty((rows, max(n, 1)), dtype=torch.int32, device=x.device)
     probs = torch.empty((rows, max(n, 1)), dtype=torch.float32, device=x.device)
     stream = torch.cuda.current_stream(x.device).cuda_stream
-    check(lib().nls_top_tokens(ctypes.c_void_p(x.data_ptr()), rows, V, n,
-                               ctypes.c_void_p(ids.data_ptr()), ctypes.c_void_p(probs.data_ptr()),
-                               ctypes.c_void_p(stream)), "nls_top_tokens")
+    work, wb = _rows_work(_ROWS_TOP_TOKENS, x, n)
+    check(lib().nls_top_tokens_ws(ctypes.c_void_p(x.data_ptr()), rows, V, n,
+                                  ctypes.c_void_p(ids.data_ptr()), ctypes.c_void_p(probs.data_ptr()),
+                                  _ptr(work), wb, ctypes.c_void_p(stream)), "nls_top_tokens")
     return ids[:, :m], probs[:, :m]
 
 
@@ -493,8 +515,10 @@ def row_nll_device(logits, targets):
     assert t.numel() == rows
     out = torch.empty(rows, dtype=torch.float64, device=x.device)
     stream = torch.cuda.current_stream(x.device).cuda_stream
-    check(lib().nls_row_nll(ctypes.c_void_p(x.data_ptr()), rows, V, ctypes.c_void_p(t.data_ptr()),
-                            ctypes.c_void_p(out.data_ptr()), ctypes.c_void_p(stream)), "nls_row_nll")
+    work, wb = _rows_work(_ROWS_NLL, x)
+    check(lib().nls_row_nll_ws(ctypes.c_void_p(x.data_ptr()), rows, V, ctypes.c_void_p(t.data_ptr()),
+                               ctypes.c_void_p(out.data_ptr()), _ptr(work), wb, ctypes.c_void_p(stream)),
+          "nls_row_nll")
     return out
 
 
@@ -511,8 +535,9 @@ def softmax_device(logits, out=None):
         out = torch.empty_like(logits)
     assert out.is_cuda and out.dtype == torch.float32 and out.is_contiguous() and out.numel() == x.numel()
     stream = torch.cuda.current_stream(x.device).cuda_stream
-    check(lib().nls_softmax_rows(ctypes.c_void_p(x.data_ptr()), rows, V, ctypes.c_void_p(out.data_ptr()),
-                                 ctypes.c_void_p(stream)), "nls_softmax_rows")
+    work, wb = _rows_work(_ROWS_SOFTMAX, x)
+    check(lib().nls_softmax_rows_ws(ctypes.c_void_p(x.data_ptr()), rows, V, ctypes.c_void_p(out.data_ptr()),
+                                    _ptr(work), wb, ctypes.c_void_p(stream)), "nls_softmax_rows")
     return out
 
 
@@ -530,9 +555,10 @@ def log_prob_device(logits, targets):
     prob = torch.empty(rows, dtype=torch.float32, device=x.device)
     logp = torch.empty(rows, dtype=torch.float64, device=x.device)
     stream = torch.cuda.current_stream(x.device).cuda_stream
-    check(lib().nls_log_prob(ctypes.c_void_p(x.data_ptr()), rows, V, ctypes.c_void_p(t.data_ptr()),
-                             ctypes.c_void_p(prob.data_ptr()), ctypes.c_void_p(logp.data_ptr()),
-                             ctypes.c_void_p(stream)), "nls_log_prob")
+    work, wb = _rows_work(_ROWS_LOG_PROB, x)
+    check(lib().nls_log_prob_ws(ctypes.c_void_p(x.data_ptr()), rows, V, ctypes.c_void_p(t.data_ptr()),
+                                ctypes.c_void_p(prob.data_ptr()), ctypes.c_void_p(logp.data_ptr()),
+                                _ptr(work), wb, ctypes.c_void_p(stream)), "nls_log_prob")
     return prob, logp
 
 

@@ -21,6 +21,7 @@
 #include "../../include/nimllm_sampler.h"
 #include "../../include/nimllm_lmhead.h"
 #include "nls_internal.h"
+#include "nls_rowsplit.h"
 
 using namespace nls;
 
@@ -1210,27 +1211,70 @@ int nls_set_rng_state(nls_sampler* s, int32_t row, uint64_t a0, uint64_t a1) {
   return NLS_OK;
 }
 
-int nls_top_tokens(const float* d_logits, int32_t rows, int64_t vocab, int32_t n, int32_t* d_ids,
-                   float* d_probs, void* stream) {
+// The workspace's kernels (nls_rowsplit.hip) when the call is one of theirs and
+// the caller brought the bytes, else the one-launch kernels: the same results.
+static bool use_split(int kind, int64_t rows, int64_t vocab, int m, const void* work, size_t work_bytes) {
+  const size_t need = nls::split_workspace(kind, rows, vocab, m);
+  return need > 0 && work && work_bytes >= need && (reinterpret_cast<uintptr_t>(work) & 15) == 0;
+}
+
+size_t nls_rows_workspace(int32_t op, int32_t rows, int64_t vocab, int32_t n) {
+  if (op < 0 || op > 3 || rows <= 0 || vocab <= 0 || (op == NLS_ROWS_TOP_TOKENS && n <= 0)) return 0;
+  return nls::split_workspace(op, rows, vocab, (int)std::min<int64_t>(n, vocab));
+}
+
+int nls_top_tokens_ws(const float* d_logits, int32_t rows, int64_t vocab, int32_t n, int32_t* d_ids,
+                      float* d_probs, void* d_work, size_t work_bytes, void* stream) {
   // (the kernel addresses a row in bytes with 32-bit offsets)
   if (rows < 0 || vocab < 0 || vocab >= (int64_t{1} << 29)) return NLS_ERR_INVALID_ARGUMENT;
   const int64_t m = std::min<int64_t>(n, vocab);  // topTokens returns min(n, len) entries (:130)
   if (rows == 0 || m <= 0) return NLS_OK;
   if (m > nls::kTopMaxN || !d_logits || !d_ids || !d_probs) return NLS_ERR_INVALID_ARGUMENT;
-  NLS_HIP(launch_top_tokens(d_logits, rows, vocab, n, d_ids, d_probs,
-                            reinterpret_cast<hipStream_t>(stream)));
+  const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (use_split(nls::kSplitTop, rows, vocab, (int)m, d_work, work_bytes)) {
+    nls::SplitArgs a{};
+    a.logits = d_logits;
+    a.V = vocab;
+    a.ids = d_ids;
+    a.probs = d_probs;
+    a.n = n;
+    a.m = (int)m;
+    NLS_HIP(nls::launch_split(nls::kSplitTop, a, rows, d_work, st));
+    return NLS_OK;
+  }
+  NLS_HIP(launch_top_tokens(d_logits, rows, vocab, n, d_ids, d_probs, st));
   return NLS_OK;
 }
 
-int nls_row_nll(const float* d_logits, int32_t rows, int64_t vocab, const int32_t* d_targets,
-                double* d_out, void* stream) {
+int nls_top_tokens(const float* d_logits, int32_t rows, int64_t vocab, int32_t n, int32_t* d_ids,
+                   float* d_probs, void* stream) {
+  return nls_top_tokens_ws(d_logits, rows, vocab, n, d_ids, d_probs, nullptr, 0, stream);
+}
+
+int nls_row_nll_ws(const float* d_logits, int32_t rows, int64_t vocab, const int32_t* d_targets, double* d_out,
+                   void* d_work, size_t work_bytes, void* stream) {
   // (the kernel addresses a row in bytes with 32-bit offsets)
   if (rows < 0 || vocab < 0 || vocab >= (int64_t{1} << 29)) return NLS_ERR_INVALID_ARGUMENT;
   if (rows == 0) return NLS_OK;
   if (vocab == 0) return NLS_ERR_EMPTY_VOCAB;
   if (!d_logits || !d_targets || !d_out) return NLS_ERR_INVALID_ARGUMENT;
-  NLS_HIP(launch_row_nll(d_logits, rows, vocab, d_targets, d_out, reinterpret_cast<hipStream_t>(stream)));
+  const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (use_split(nls::kSplitNll, rows, vocab, 0, d_work, work_bytes)) {
+    nls::SplitArgs a{};
+    a.logits = d_logits;
+    a.V = vocab;
+    a.targets = d_targets;
+    a.logp = d_out;
+    NLS_HIP(nls::launch_split(nls::kSplitNll, a, rows, d_work, st));
+    return NLS_OK;
+  }
+  NLS_HIP(launch_row_nll(d_logits, rows, vocab, d_targets, d_out, st));
   return NLS_OK;
+}
+
+int nls_row_nll(const float* d_logits, int32_t rows, int64_t vocab, const int32_t* d_targets,
+                double* d_out, void* stream) {
+  return nls_row_nll_ws(d_logits, rows, vocab, d_targets, d_out, nullptr, 0, stream);
 }
 
 int nls_argmax(const float* d_logits, int32_t rows, int64_t vocab, int32_t* d_out, void* stream) {
@@ -1242,25 +1286,54 @@ int nls_argmax(const float* d_logits, int32_t rows, int64_t vocab, int32_t* d_ou
   return NLS_OK;
 }
 
-int nls_softmax_rows(const float* d_logits, int32_t rows, int64_t vocab, float* d_out, void* stream) {
+int nls_softmax_rows_ws(const float* d_logits, int32_t rows, int64_t vocab, float* d_out, void* d_work,
+                        size_t work_bytes, void* stream) {
   // (the kernel addresses a row in bytes with 32-bit offsets)
   if (rows < 0 || vocab < 0 || vocab >= (int64_t{1} << 29)) return NLS_ERR_INVALID_ARGUMENT;
   if (rows == 0) return NLS_OK;
   if (vocab == 0) return NLS_ERR_EMPTY_VOCAB;
   if (!d_logits || !d_out) return NLS_ERR_INVALID_ARGUMENT;
-  NLS_HIP(launch_softmax_rows(d_logits, rows, vocab, d_out, reinterpret_cast<hipStream_t>(stream)));
+  const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (use_split(nls::kSplitSoftmax, rows, vocab, 0, d_work, work_bytes)) {
+    nls::SplitArgs a{};
+    a.logits = d_logits;
+    a.V = vocab;
+    a.out = d_out;
+    NLS_HIP(nls::launch_split(nls::kSplitSoftmax, a, rows, d_work, st));
+    return NLS_OK;
+  }
+  NLS_HIP(launch_softmax_rows(d_logits, rows, vocab, d_out, st));
+  return NLS_OK;
+}
+
+int nls_softmax_rows(const float* d_logits, int32_t rows, int64_t vocab, float* d_out, void* stream) {
+  return nls_softmax_rows_ws(d_logits, rows, vocab, d_out, nullptr, 0, stream);
+}
+
+int nls_log_prob_ws(const float* d_logits, int32_t rows, int64_t vocab, const int32_t* d_targets, float* d_prob,
+                    double* d_logp, void* d_work, size_t work_bytes, void* stream) {
+  if (rows < 0 || vocab < 0 || vocab >= (int64_t{1} << 29)) return NLS_ERR_INVALID_ARGUMENT;
+  if (rows == 0) return NLS_OK;
+  if (vocab == 0) return NLS_ERR_EMPTY_VOCAB;
+  if (!d_logits || !d_targets || !d_prob || !d_logp) return NLS_ERR_INVALID_ARGUMENT;
+  const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (use_split(nls::kSplitLogProb, rows, vocab, 0, d_work, work_bytes)) {
+    nls::SplitArgs a{};
+    a.logits = d_logits;
+    a.V = vocab;
+    a.targets = d_targets;
+    a.prob = d_prob;
+    a.logp = d_logp;
+    NLS_HIP(nls::launch_split(nls::kSplitLogProb, a, rows, d_work, st));
+    return NLS_OK;
+  }
+  NLS_HIP(launch_log_prob(d_logits, rows, vocab, d_targets, d_prob, d_logp, st));
   return NLS_OK;
 }
 
 int nls_log_prob(const float* d_logits, int32_t rows, int64_t vocab, const int32_t* d_targets, float* d_prob,
                  double* d_logp, void* stream) {
-  if (rows < 0 || vocab < 0 || vocab >= (int64_t{1} << 29)) return NLS_ERR_INVALID_ARGUMENT;
-  if (rows == 0) return NLS_OK;
-  if (vocab == 0) return NLS_ERR_EMPTY_VOCAB;
-  if (!d_logits || !d_targets || !d_prob || !d_logp) return NLS_ERR_INVALID_ARGUMENT;
-  NLS_HIP(launch_log_prob(d_logits, rows, vocab, d_targets, d_prob, d_logp,
-                          reinterpret_cast<hipStream_t>(stream)));
-  return NLS_OK;
+  return nls_log_prob_ws(d_logits, rows, vocab, d_targets, d_prob, d_logp, nullptr, 0, stream);
 }
 
 int nls_expf_device(const float* d_in, float* d_out, int64_t n, void* stream) {

@@ -158,6 +158,43 @@ NLS_HD inline float expf_hard_lookup(float x, float fallback) {
   return fallback;
 }
 
+// The table form without its special cases, for x in [-87, 0] (results in the
+// normal range): the correctly rounded e^x where `ok`; where the float64
+// value lies within 2^-47 of a rounding boundary, or x is anything else, `ok`
+// is false and the result means nothing.  k comes from the low word of
+// x 64/ln2 + 1.5 2^52, 2^(k >> 6) is added to the table entry's exponent field, and
+// the boundary is looked for in the 29 bits that the rounding drops: 21
+// operations where expf_cr_t takes about 35.
+NLS_HD inline float expf_cr_quick(float xf, const double* pow2, bool& ok) {
+  const double x = (double)xf;
+  const double kInvStep = 0x1.71547652b82fep+6;
+  const double kStepHi = 0x1.62e42fefa0000p-7;
+  const double kStepLo = 0x1.cf79abc9e3b3ap-46;
+  const double kMagic = 0x1.8p+52;
+  const double km = __builtin_fma(x, kInvStep, kMagic);
+  uint64_t kb;
+  memcpy(&kb, &km, sizeof kb);
+  const uint32_t k = (uint32_t)kb;  // two's complement
+  const double kd = km - kMagic;
+  double r = __builtin_fma(-kd, kStepHi, x);
+  r = __builtin_fma(-kd, kStepLo, r);
+  double u = __builtin_fma(0x1.1111111111111p-7, r, 0x1.5555555555555p-5);
+  u = __builtin_fma(u, r, 0x1.5555555555555p-3);
+  u = __builtin_fma(u, r, 0.5);
+  const double q = __builtin_fma(u, r * r, r);
+  double t = pow2[k & (kExpfPow2Count - 1)];
+  uint64_t tb;
+  memcpy(&tb, &t, sizeof tb);
+  tb = (tb & 0xffffffffull) | ((uint64_t)((uint32_t)(tb >> 32) + ((k & ~63u) << 14)) << 32);
+  memcpy(&t, &tb, sizeof t);
+  const double y = __builtin_fma(t, q, t);
+  uint64_t yb;
+  memcpy(&yb, &y, sizeof yb);
+  // 2^-47 of y is at most 2^6 units of its last place
+  ok = xf >= -87.0f && (((uint32_t)yb - ((1u << 28) - 64u)) & 0x1fffffffu) > 128u;
+  return (float)y;
+}
+
 // Correctly rounded e^x for binary32 x.
 NLS_HD inline float expf_cr(float x) {
   if (!(x > -104.0f)) {            // exp(-104) < 2^-150: rounds to +0

@@ -11,6 +11,7 @@
 // with -ffp-contract=off so no multiply-add is fused.
 #include "nls_device.h"
 #include "nls_launch.h"
+#include "nls_rowsplit.h"
 #include "nls_seqsum.h"
 
 namespace nls {
@@ -52,10 +53,16 @@ constexpr int kTopCh = kTopThreads * kTopPer;   // 8192 exponentials in LDS
 constexpr int kTopList = 2048;                  // logits listed at or above the bound
 }  // namespace
 
-template <int NT>
+//
+// PRE: rows split over workgroups (nls_rowsplit.hip) arrive with mx, s and the
+// listed entries; steps 1 and 2 are theirs.  A list of up to 1024 entries is
+// ordered by counting, for each entry, the entries before it.
+template <int NT, bool PRE>
 __global__ __launch_bounds__(NT) void top_tokens_kernel(const float* __restrict__ logits, int64_t V,
                                                         int n, int32_t* __restrict__ ids,
-                                                        float* __restrict__ probs) {
+                                                        float* __restrict__ probs,
+                                                        const SplitRowInfo* __restrict__ pre_info,
+                                                        const uint64_t* __restrict__ pre_list) {
   constexpr int NW = NT / kWave;
   static_assert((size_t)kTopCh * sizeof(float) >= (size_t)kTopMaxN * 2 * sizeof(uint64_t),
                 "the members (and the fallback's candidates) reuse the exponentials' buffer");
@@ -125,9 +132,23 @@ __global__ __launch_bounds__(NT) void top_tokens_kernel(const float* __restrict_
     }
   };
 
+  float mx = -__builtin_inff();
+  float s = 0.0f;
+  uint32_t t0 = 0u;  // every entry whose logit key is at least t0 is listed
+  int nl;
+  if constexpr (PRE) {
+    static_assert(kSplitList == kTopList, "the list's capacity");
+    const SplitRowInfo& in = pre_info[row];
+    mx = in.mx;
+    s = in.sum;
+    nl = in.count;
+    t0 = f2key(in.bound);
+    if (tid < kExpfPow2Count) s_pow2[tid] = kExpfPow2J64[tid];
+    for (int i = tid; i < min(nl, kTopList); i += NT) list[i] = pre_list[(int64_t)row * kTopList + i];
+    __syncthreads();
+  } else {
   // (1) mx and each thread's largest logit key (the next chunk requested
   // before the current one is reduced)
-  float mx = -__builtin_inff();
   uint32_t tk = 0u;
   {
     float a[kTopPer], b[kTopPer];
@@ -156,7 +177,6 @@ __global__ __launch_bounds__(NT) void top_tokens_kernel(const float* __restrict_
   for (int w = 1; w < NW; ++w) mx = __builtin_fmaxf(mx, s_part[w]);
   // the bound: the m-th largest thread maximum, when at least m threads hold
   // an element (else every element is listed)
-  uint32_t t0 = 0u;
   const int holders = vec ? min(NT, (nV + 3) / 4) : min(NT, nV);
   if (m <= holders) {
     const SelectResult b0 = block_select<NT>([&](auto fn) { fn(tk, tid < holders); }, m, -1, hist, smem);
@@ -167,7 +187,6 @@ __global__ __launch_bounds__(NT) void top_tokens_kernel(const float* __restrict_
   __syncthreads();
 
   // (2) s = e_0 + e_1 + ... in index order (:54-56), listing the logits >= t0
-  float s = 0.0f;
   {
     int J = 1, nwin = 0;
     float v[kTopPer];
@@ -190,7 +209,8 @@ __global__ __launch_bounds__(NT) void top_tokens_kernel(const float* __restrict_
       s = seq_sum_block<NT>(ebuf, min(kTopCh, nV - c0), s, J, nwin, c0, sh);  // ends with a barrier
     }
   }
-  const int nl = s_cnt;
+  nl = s_cnt;
+  }
   // probs[i] /= s (:57)
   auto prob_of = [&](float l) -> float { return expf_cr_t(l - mx, s_pow2) / s; };
   auto pkey = [&](float l) -> uint32_t { return f2key(prob_of(l)); };
@@ -209,6 +229,33 @@ __global__ __launch_bounds__(NT) void top_tokens_kernel(const float* __restrict_
       probs[(int64_t)row * n + j] = key2f((uint32_t)(e >> 32));
     }
   };
+  if constexpr (PRE) {
+    if (s == s && nl >= m && nl <= NT) {  // uniform
+      uint64_t mine = 0ull;
+      if (tid < nl) {
+        const uint64_t le = list[tid];
+        mine = ((uint64_t)pkey(key2f((uint32_t)(le >> 32))) << 32) | (0xffffffffu - (uint32_t)le);
+        mem[tid] = mine;
+      }
+      __syncthreads();
+      int rank = 0;
+      if (tid < nl)
+        for (int i = 0; i < nl; ++i) rank += mem[i] > mine;
+      // unlisted entries lie below t0: out of the first m when the largest
+      // logit they could have falls short of the m-th probability
+      if (tid < nl && rank == m - 1)
+        smem[0] = t0 == f2key(-__builtin_inff()) || pkey(key2f(t0 - 1u)) < (uint32_t)(mine >> 32);
+      __syncthreads();
+      if (smem[0]) {
+        if (tid < nl && rank < m) {
+          ids[(int64_t)row * n + rank] = (int32_t)(0xffffffffu - (uint32_t)mine);
+          probs[(int64_t)row * n + rank] = key2f((uint32_t)(mine >> 32));
+        }
+        return;
+      }
+      __syncthreads();
+    }
+  }
   // the lowest key in [key(-inf), key(L)] whose probability reaches p(L)
   auto lowest_key = [&](uint32_t kL) -> uint32_t {
     const float pm = prob_of(key2f(kL));
@@ -547,9 +594,9 @@ __global__ void generate_step_kernel(const int32_t* __restrict__ out, int B, int
   hist_len[b] = len + 1;
 }
 
-// Both device evaluations of the exponential: y[i] = exp(x[i]) when they
-// agree, else a NaN with the payload 0xdead (so a checksum over every input
-// covers both).
+// Every device evaluation of the exponential: y[i] = exp(x[i]) when the two
+// exact ones agree, the quick one where it holds, and the estimate keeps its bound, else a NaN with the
+// payload 0xdead (so a checksum over every input covers all).
 __global__ void expf_kernel(const float* __restrict__ x, float* __restrict__ y, int64_t n) {
   __shared__ double pow2[kExpfPow2Count];
   if (threadIdx.x < kExpfPow2Count) pow2[threadIdx.x] = kExpfPow2J64[threadIdx.x];
@@ -558,7 +605,15 @@ __global__ void expf_kernel(const float* __restrict__ x, float* __restrict__ y, 
   if (i < n) {
     const float a = expf_cr(x[i]);
     const float b = expf_cr_t(x[i], pow2);
-    y[i] = __float_as_uint(a) == __float_as_uint(b) ? a : __uint_as_float(0x7fc0deadu);
+    bool same = __float_as_uint(a) == __float_as_uint(b);
+    if (x[i] <= 0.0f) {
+      const float est = expf_estimate(x[i]);
+      bool ok;
+      const float c = expf_cr_quick(x[i], pow2, ok);
+      same = same && (!ok || __float_as_uint(a) == __float_as_uint(c));
+      same = same && (x[i] >= -87.0f ? __builtin_fabsf(est - a) <= a * kSplitErr : est >= 0.0f && est < 0x1p-125f);
+    }
+    y[i] = same ? a : __uint_as_float(0x7fc0deadu);
   }
 }
 
@@ -646,8 +701,14 @@ hipError_t set_kernel_attributes() {
 
 hipError_t launch_top_tokens(const float* logits, int rows, int64_t V, int n, int32_t* ids,
                              float* probs, hipStream_t s) {
-  hipLaunchKernelGGL(top_tokens_kernel<kTopThreads>, dim3(rows), dim3(kTopThreads), 0, s, logits, V, n,
-                     ids, probs);
+  hipLaunchKernelGGL((top_tokens_kernel<kTopThreads, false>), dim3(rows), dim3(kTopThreads), 0, s, logits, V, n,
+                     ids, probs, nullptr, nullptr);
+  return hipGetLastError();
+}
+
+hipError_t launch_split_top(const SplitArgs& a, int rows, hipStream_t s) {
+  hipLaunchKernelGGL((top_tokens_kernel<kTopThreads, true>), dim3(rows), dim3(kTopThreads), 0, s, a.logits, a.V,
+                     a.n, a.ids, a.probs, a.info, a.list);
   return hipGetLastError();
 }
 
