@@ -898,6 +898,128 @@ __global__ __launch_bounds__(kLmNT) void lm_float_kernel(FloatArgs a) {
   }
 }
 
+// dotF32 of F16 / BF16 rows.  Eight consecutive weights hold one element of
+// each of the eight chains, so a 16-byte piece needs no exchange between lanes
+// once it sits in the lanes that own the row: P lanes, 8 / P chains each.  A
+// wave reads 8 KB of its 64 / P rows at a time, 128 P contiguous bytes per row, one
+// tile ahead of its use, and turns it through LDS (rows padded by 16 bytes:
+// no bank conflicts); the activations stand in LDS in the order they come.
+// Bound: HBM.  lm_float_kernel, whose lanes own one chain each, moves every
+// weight through LDS as a float of its own, in and out, 64 weights of a row at
+// a time.  F16, one state, lm_float_kernel -> here: 128256 x 2048 179 -> 101 us
+// (5.2 TB/s), 32000 x 4096 86 -> 45, 8000 x 1024 17.5 -> 9.0; four states of 128256 x
+// 2048 543 -> 145.  (P = 1, the activations through the scalar cache: 107 us,
+// and 235 for four states.)
+template <int P>
+constexpr int half_lds_wave() {
+  return (64 / P) * (128 * P + 16);
+}
+template <int T>
+__device__ __forceinline__ float half_value(uint32_t pair, int hi) {
+  if constexpr (T == 1) return lm_half_f(hi ? pair >> 16 : pair & 0xFFFF);
+  return __uint_as_float(hi ? pair & 0xFFFF0000u : pair << 16);
+}
+
+template <int T, int P, int NB>
+__global__ __launch_bounds__(kLmNT) void lm_half_kernel(FloatArgs a) {
+  static_assert(T == 1 || T == 30, "two-byte weights");
+  static_assert(P == 2 || P == 4, "lanes per row");
+  constexpr int R = 64 / P;        // rows per wave
+  constexpr int C = 8 / P;         // chains per lane
+  constexpr int PC = 8 * P;        // 16-byte pieces of a row per tile
+  constexpr int PITCH = 128 * P + 16;
+  extern __shared__ __align__(16) uint8_t lds[];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  uint8_t* tile = lds + wv * half_lds_wave<P>();
+  float* xl = reinterpret_cast<float*>(lds + (kLmNT / 64) * half_lds_wave<P>());  // [NB][c8]
+  const int64_t r0 = ((int64_t)blockIdx.x * (kLmNT / 64) + wv) * R;
+  const int c8 = (int)(a.cols & ~(int64_t)7);
+  const int pieces = c8 / 8;  // per row
+  for (int b = 0; b < NB; ++b)
+    for (int i = threadIdx.x; i < c8; i += kLmNT) xl[b * c8 + i] = a.x[(int64_t)b * a.cols + i];
+  __syncthreads();
+  if (r0 >= a.rows) return;
+  // load i of a tile: piece lane % PC of row i * (64 / PC) + lane / PC
+  const uint8_t* src[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    src[i] = a.w + min(r0 + i * (64 / PC) + lane / PC, a.rows - 1) * a.row_bytes + 16 * (lane % PC);
+  uint4 nxt[8];
+  auto request = [&](int pc) __attribute__((always_inline)) {
+    const bool in = pc + lane % PC < pieces;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (in) nxt[i] = lm_ld_16(src[i] + 16 * (int64_t)pc);
+  };
+  const int row = lane / P, part = lane % P;
+  float acc[NB][C];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int c = 0; c < C; ++c) acc[b][c] = 0.0f;
+  // piece q of the tile at pc: its C weights of this lane's chains
+  auto piece = [&](int pc, int q) __attribute__((always_inline)) {
+    uint32_t u[C / 2];
+    __builtin_memcpy(u, __builtin_assume_aligned(tile + row * PITCH + 16 * q + part * (16 / P), 16 / P), 16 / P);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      float xv[C];
+      __builtin_memcpy(xv, __builtin_assume_aligned(xl + b * c8 + 8 * (pc + q) + part * C, 4 * C), 4 * C);
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+        acc[b][c] = __fadd_rn(acc[b][c], __fmul_rn(half_value<T>(u[c >> 1], c & 1), xv[c]));
+    }
+  };
+  request(0);
+  for (int pc = 0; pc < pieces; pc += PC) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      *reinterpret_cast<uint4*>(tile + (i * (64 / PC) + lane / PC) * PITCH + 16 * (lane % PC)) = nxt[i];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (pc + PC < pieces) request(pc + PC);
+    if (pc + PC <= pieces) {
+#pragma unroll
+      for (int q = 0; q < PC; ++q) piece(pc, q);
+    } else {
+      for (int q = 0; q < pieces - pc; ++q) piece(pc, q);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+  const int64_t r = r0 + row;
+  if (part == 0) {  // the tail goes to chain 0
+    const uint8_t* rp = a.w + min(r, a.rows - 1) * a.row_bytes;
+    for (int64_t e = c8; e < a.cols; ++e) {
+      const float w = deq1<T>(rp, e);
+#pragma unroll
+      for (int b = 0; b < NB; ++b) acc[b][0] = __fadd_rn(acc[b][0], __fmul_rn(w, a.x[(int64_t)b * a.cols + e]));
+    }
+  }
+  // ((p01 + p23) + p45) + p67, left to right (quant.nim:374)
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    float pr[C / 2];
+#pragma unroll
+    for (int c = 0; c < C / 2; ++c) pr[c] = __fadd_rn(acc[b][2 * c], acc[b][2 * c + 1]);
+    float t = pr[0];
+#pragma unroll
+    for (int c = 1; c < C / 2; ++c) t = __fadd_rn(t, pr[c]);  // (lane 0's share of the chain)
+#pragma unroll
+    for (int k = 1; k < P; ++k) {
+      const float below = __shfl(t, (lane & ~(P - 1)) + k - 1);
+      if (part == k) {
+        t = __fadd_rn(below, pr[0]);
+#pragma unroll
+        for (int c = 1; c < C / 2; ++c) t = __fadd_rn(t, pr[c]);
+      }
+    }
+    if (part == P - 1 && r < a.rows) a.y[(int64_t)b * a.rows + r] = t;
+  }
+}
+
 // ------------------------------------------------ LoRA (model.nim:189-200)
 
 // tmp[b, i] = dotF32(A[i, :], x[b, :]): one group of 8 lanes per (b, i).
@@ -1020,8 +1142,54 @@ hipError_t launch_int(const LmHeadCall& c, hipStream_t s) {
   else return launch_int32<T>(c, nblk, passes, s);
 }
 
+template <int T, int P, int NB>
+hipError_t launch_half(const FloatArgs& a, int64_t c8, hipStream_t s) {
+  const int64_t per = (kLmNT / 64) * (64 / P);
+  const size_t lds = (kLmNT / 64) * half_lds_wave<P>() + (size_t)NB * (size_t)c8 * 4;
+  if (lds > 65536) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(lm_half_kernel<T, P, NB>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL((lm_half_kernel<T, P, NB>), dim3((unsigned)((a.rows + per - 1) / per)), dim3(kLmNT), lds, s, a);
+  return hipGetLastError();
+}
+template <int T, int P>
+hipError_t launch_half_states(const FloatArgs& a, int64_t c8, hipStream_t s) {
+  switch (a.nb) {
+    case 1: return launch_half<T, P, 1>(a, c8, s);
+    case 2: return launch_half<T, P, 2>(a, c8, s);
+    case 3: return launch_half<T, P, 3>(a, c8, s);
+    default: return launch_half<T, P, 4>(a, c8, s);
+  }
+}
+
+// Activations of a pass of lm_half_kernel (with its tiles, 100 KB of LDS).
+constexpr int64_t kHalfActBytes = 65536;
+
 template <int T>
 hipError_t launch_float(const LmHeadCall& c, hipStream_t s) {
+  if constexpr (T == 1 || T == 30) {
+    const int64_t c8 = c.cols & ~(int64_t)7;
+    if (c8 > 0 && c8 * 4 <= kHalfActBytes) {
+      const int pass = (int)std::min<int64_t>(kLmNBC, kHalfActBytes / (c8 * 4));
+      for (int b0 = 0; b0 < c.nb; b0 += pass) {
+        const int nb = std::min(c.nb - b0, pass);
+        const FloatArgs a{static_cast<const uint8_t*>(c.w), c.rows, c.cols, c.row_bytes,
+                          c.x + (int64_t)b0 * c.cols, nb, c.y + (int64_t)b0 * c.rows};
+        // P = 4 keeps more waves per row; P = 2 reads the activations in half as
+        // many LDS operations, which counts from three states on (128256 x 2048,
+        // four states: 145 us against 169; 16000 x 4096, too few rows for it: 97
+        // against 69), and takes half as many workgroups, which counts where
+        // these fill one round of three per CU and P = 4's start a second
+        // (50001 x 2048: 32 us against 38; 98304 x 2048: 90 against 81)
+        const bool two = nb >= 3 ? c.rows >= 32768 : c.rows > 49152 && c.rows <= 81920;
+        const hipError_t e = two ? launch_half_states<T, 2>(a, c8, s) : launch_half_states<T, 4>(a, c8, s);
+        if (e != hipSuccess) return e;
+      }
+      return hipSuccess;
+    }
+  }
   FloatArgs a{static_cast<const uint8_t*>(c.w), c.rows, c.cols, c.row_bytes, c.x, c.nb, c.y};
   const int64_t grid = (c.rows + kLmNT / 8 - 1) / (kLmNT / 8);
   // the activations of a pass in LDS when they fit in 32 KiB

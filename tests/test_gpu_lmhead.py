@@ -251,3 +251,20 @@ def test_batched_states_parity(pkg, name):
     want = O.matmul(t, w, rows, cols, x)
     got = pkg.lm_head(torch.from_numpy(w).cuda(), t, rows, cols, torch.from_numpy(x).cuda()).cpu().numpy()
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["F16", "BF16"])
+def test_half_weights_parity(pkg, name):
+    """Two-byte weights around the edges of their kernel: rows around a wave's
+    16 or 32 and a workgroup's 64 or 128, columns around one tile (128 or 256)
+    with and without a tail, odd row starts, and the row, state and column
+    counts where the lanes per row and the states per pass change: every logit
+    bit for bit."""
+    t = TYPES[name]
+    cases = [(1, 7, 1), (1, 8, 1), (15, 9, 2), (17, 255, 1), (63, 256, 3), (64, 257, 4), (65, 263, 1), (31, 264, 2),
+             (130, 519, 5), (300, 1000, 1), (40, 8192, 3), (20, 16384, 5), (20, 16392, 1),
+             (32767, 40, 3), (32769, 136, 3), (32800, 72, 4), (49152, 24, 1), (49153, 129, 1), (81921, 33, 2)]
+    for rows, cols, nb in cases:
+        print(f"lm_head two-byte {name} rows={rows} cols={cols} nb={nb}", flush=True)
+        run_case(pkg, t, rows, cols, nb, seed=rows + cols)
