@@ -158,6 +158,12 @@ struct nls_sampler {
   // counters it would have handed on are cleared before the next call
   bool counters_dirty = false;
   int hbits = 0;   // k64_kernel's hash table: 2^hbits slots
+  // Fewer rows than CUs with windows that may outgrow that table: the split
+  // rows' plan, for the calls whose windows may have (S > 1: there is one).
+  struct SplitPlan {
+    int S = 1, L = 0, xcd_map = 0, ccap = 0, nwords = 0, pcap = 0, mcap = 0, kcap = 0, offA = 0, pc = 0, nt = 0, q = 0;
+    size_t lds = 0;
+  } alt;
 
   RowParams* rp = nullptr;
   int32_t* bias_ids = nullptr;
@@ -253,8 +259,12 @@ struct nls_sampler {
   // (history window + bias entries) than its LDS table holds: such a row is
   // handed on to the whole-row path, which then gets a launch of its own
   // across the CUs rather than the streaming kernel's last workgroup.
+  int64_t k64_patches() const { return (int64_t)((1 << hbits) - (1 << hbits) / 4); }
+  bool split_now() const { return alt.S > 1 && windows_exceed(k64_patches()); }
   bool window_may_overflow() const {
-    const int64_t cap = plan.k64 ? (int64_t)((1 << hbits) - (1 << hbits) / 4) : (int64_t)pcap;
+    return windows_exceed(split_now() ? alt.pcap : plan.k64 ? k64_patches() : (int64_t)pcap);
+  }
+  bool windows_exceed(int64_t cap) const {
     for (int b = 0; b < B; ++b) {
       const RowParams& r = h_rp[b];
       if (!r.fast) continue;
@@ -335,7 +345,23 @@ struct Geometry {
   size_t lds;
 };
 
-Geometry plan_geometry(int B, int64_t V, int kmax, int ncu, int max_patch) {
+// Whether a batch of fewer rows than CUs still streams each row in one
+// workgroup.  k64_kernel's one workgroup has no candidates to exchange, and
+// its serial phases are shorter: sampled at k = 40, 1 x 128256 29 us against 38 split,
+// 24 x 50001 27.5 against 30.6, 200 x 128256 32 against 97, 1 x 262144 46 against 53.  A
+// greedy row has nothing to exchange but its maximum, so few long ones are
+// split (1 x 128256: 14.3 against 15.7, 8 x 200000: 17.8 against 19.5; 64 x 128256: 33
+// against 16).  Past 262144 ids the bitmap leaves too little LDS to the patch
+// table; k > 64 streams whole rows at a workgroup's pace and stays split.
+// (Small batches of greedy beside top-k rows and no full sorts, `both`, also
+// stay: their split plan is the one the tests of NaN rows over slices expect.)
+bool whole_rows(int B, int64_t V, int kmax, int ncu, bool both) {
+  if (B >= ncu || V <= kSmallRowV) return true;
+  if (kmax > kWaveTopK || V > kWholeRowV || both) return false;
+  return kmax > 0 || V <= kWholeGreedyV || B >= kWholeGreedyRows;
+}
+
+Geometry plan_geometry(int B, int64_t V, int kmax, int ncu, int max_patch, bool whole) {
   Geometry g{};
   // Top-k rows past the wave path (k > 64) on a batch of at least two rows
   // per CU: 512-thread workgroups whose LDS leaves room for two per CU, so
@@ -362,14 +388,10 @@ Geometry plan_geometry(int B, int64_t V, int kmax, int ncu, int max_patch) {
     d.lds = cand + std::max(head + (size_t)d.pcap * 16, tail);
     if (d.lds <= target && d.pcap >= std::max(max_patch, 1)) return d;
   }
-  // 256-thread workgroups, >= 4 per CU: rows are split into S slices until the
-  // grid holds about 4 workgroups per CU, keeping >= 2 tiles per slice.
-  // a whole row per 1024-thread workgroup once the batch fills the chip, or
-  // when a row is small enough that one workgroup streams it faster than the
-  // slices of a split row exchange their candidates (V = 32000, B = 1: 18.9
-  // against 23.9 us per call); otherwise rows are split over 256-thread
-  // workgroups
-  g.nt = env_int("NLS_STREAM_NT", (B >= ncu || V <= kSmallRowV) ? 1024 : 256) == 1024 ? 1024 : 256;
+  // A whole row per 1024-thread workgroup (whole_rows), else rows are split
+  // into S slices of 256-thread workgroups until the grid holds about 4 per CU,
+  // keeping >= 2 tiles per slice.
+  g.nt = env_int("NLS_STREAM_NT", whole ? 1024 : 256) == 1024 ? 1024 : 256;
   const int64_t te = (int64_t)g.nt * kStreamVec4 * 4;
   const int want = g.nt == 1024 ? 1 : std::max(1, (4 * ncu + B - 1) / B);
   g.S = std::max(1, env_int("NLS_STREAM_S", want));
@@ -557,10 +579,20 @@ int nls_create(const nls_params* per_row, int32_t batch, int64_t vocab, void* st
   if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1)
     ncu = 256;
   int kfast = kmax;
-  Geometry g = plan_geometry(B, vocab, kfast, ncu, max_patch);
+  bool both = false;
+  {
+    bool greedy = false, topk = false, full = false;
+    for (int b = 0; b < B; ++b) {
+      const RowParams& r = s->h_rp[b];
+      greedy |= r.mode == kModeGreedy;
+      (r.mode == kModeTopK && r.k <= kMaxTopKFast ? topk : full) |= r.mode != kModeGreedy;
+    }
+    both = greedy && topk && !full;
+  }
+  Geometry g = plan_geometry(B, vocab, kfast, ncu, max_patch, whole_rows(B, vocab, kfast, ncu, both));
   while (kfast > 0 && (g.lds > max_dynamic_lds() || (g.nt != 512 && g.pcap < 256))) {
     kfast = kfast * 7 / 8;
-    g = plan_geometry(B, vocab, kfast, ncu, max_patch);
+    g = plan_geometry(B, vocab, kfast, ncu, max_patch, whole_rows(B, vocab, kfast, ncu, both));
   }
   // (false only for vocabularies far beyond 2^19; the slice's byte size must
   // also fit the 32-bit range of the kernel's buffer loads)
@@ -607,6 +639,28 @@ int nls_create(const nls_params* per_row, int32_t batch, int64_t vocab, void* st
         any_topk |= s->h_rp[b].mode == kModeTopK;
       }
       if (any_greedy != any_topk) s->plan.k64_rows = any_greedy ? kK64RowsGreedy : kK64RowsTopK;
+      // the split rows' plan beside it where a window may outgrow the table
+      // (a row past it takes the whole-row path, milliseconds; the slices of a
+      // split row hold a table each)
+      if (B < ncu && vocab > kSmallRowV && (max_patch < 0 || max_patch > s->k64_patches())) {
+        const Geometry d = plan_geometry(B, vocab, kfast, ncu, max_patch, false);
+        if (d.S > 1 && d.wave && d.nt == 256 && d.lds <= max_dynamic_lds() && d.pcap >= 256) {
+          auto& t = s->alt;
+          t.S = d.S;
+          t.L = d.L;
+          t.xcd_map = B % 8 == 0 ? 1 : 0;
+          t.ccap = d.ccap;
+          t.nwords = d.nwords;
+          t.pcap = d.pcap;
+          t.mcap = d.mcap;
+          t.kcap = d.kcap;
+          t.offA = d.offA;
+          t.pc = d.pc;
+          t.nt = d.nt;
+          t.q = d.q;
+          t.lds = d.lds;
+        }
+      }
     }
   }
   // Without full-sort rows the whole-row kernel only serves the rare row the
@@ -664,9 +718,10 @@ int nls_create(const nls_params* per_row, int32_t batch, int64_t vocab, void* st
   if ((rc = dalloc(&s->bias_ids, std::max<size_t>(bid.size(), 1)))) return fail(rc);
   if ((rc = dalloc(&s->bias_vals, std::max<size_t>(bval.size(), 1)))) return fail(rc);
   if ((rc = dalloc(&s->hist_len, B))) return fail(rc);
-  if (s->S > 1) {
-    if ((rc = dalloc(&s->part_cand, (size_t)B * s->S * s->pc))) return fail(rc);
-    if ((rc = dalloc(&s->part_info, (size_t)B * s->S))) return fail(rc);
+  if (s->S > 1 || s->alt.S > 1) {
+    const int S = s->S > 1 ? s->S : s->alt.S, pc = s->S > 1 ? s->pc : s->alt.pc;
+    if ((rc = dalloc(&s->part_cand, (size_t)B * S * pc))) return fail(rc);
+    if ((rc = dalloc(&s->part_info, (size_t)B * S))) return fail(rc);
   }
   if ((rc = dalloc(&s->arrive, B))) return fail(rc);
   if ((rc = dalloc(&s->rng, (size_t)2 * B))) return fail(rc);
@@ -963,6 +1018,24 @@ int sample_impl(nls_sampler* s, const float* d_logits, const double* d_u, int32_
     }
   }
   LaunchPlan lp = s->plan;
+  const bool split_now = s->split_now();
+  if (split_now) {
+    const auto& t = s->alt;
+    a.S = t.S;
+    a.L = t.L;
+    a.xcd_map = t.xcd_map;
+    a.ccap = t.ccap;
+    a.nwords = t.nwords;
+    a.pcap = t.pcap;
+    a.mcap = t.mcap;
+    a.kcap = t.kcap;
+    a.offA = t.offA;
+    a.pc = t.pc;
+    lp.k64 = false;
+    lp.nt = t.nt;
+    lp.q = t.q;
+    lp.lds = t.lds;
+  }
   a.gen_inline = s->gen_inline;
   if (a.gen_inline && s->window_may_overflow()) {
     const int want = std::min(s->B, s->ncu);
@@ -1020,7 +1093,7 @@ int sample_impl(nls_sampler* s, const float* d_logits, const double* d_u, int32_
     ga.next_count = s->all_rows + s->B + 1;
     a.gen_inline = 0;
   }
-  if (s->k64_list && !lp.no_stream) {
+  if (s->k64_list && !lp.no_stream && !split_now) {
     a.row_list = s->k64_list;
     a.n_list = s->n_k64_list;
     ga.fixed_list = s->full_list;
@@ -1089,16 +1162,18 @@ int nls_profile_next_generic(nls_sampler* s, void* start_event, void* stop_event
 int nls_get_plan(const nls_sampler* s, nls_plan* out, int32_t* row_streamed) {
   if (!s || !out) return NLS_ERR_INVALID_ARGUMENT;
   std::memset(out, 0, sizeof *out);
-  out->stream_threads = s->plan.lds > 0 ? s->plan.nt : 0;
-  out->slices = s->S;
+  const bool split = s->split_now();
+  const int nt = split ? s->alt.nt : s->plan.nt, S = split ? s->alt.S : s->S;
+  out->stream_threads = s->plan.lds > 0 ? nt : 0;
+  out->slices = S;
   out->generic_launch = s->gen_inline ? 0 : 1;
-  out->k64 = s->plan.k64 ? 1 : 0;
+  out->k64 = s->plan.k64 && !split ? 1 : 0;
   out->walk_split = s->walk_split ? 1 : 0;
   out->floor_slices = s->plan.floor_slices;
   // a workgroup requests its first unit (kStreamVec4 float4 per thread)
   // before it reads the row's constants
   out->first_unit_bytes = (s->plan.lds > 0 && !s->plan.no_stream)
-                              ? std::min<int64_t>((int64_t)s->S * s->plan.nt * kStreamVec4 * 16, s->V * 4)
+                              ? std::min<int64_t>((int64_t)S * nt * kStreamVec4 * 16, s->V * 4)
                               : 0;
   for (int b = 0; b < s->B; ++b) {
     const int f = s->h_rp[b].fast ? 1 : 0;

@@ -1632,3 +1632,53 @@ def test_generate_step_every_path(pkg, torch, B, V, ks):
         assert any(done) and not all(done)
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("B,V,off", [(1, 50001, 0), (9, 128256, 1), (24, 65536, 0), (3, 262144, 0), (2, 262145, 0)])
+def test_windows_that_outgrow_the_patch_table(pkg, torch, B, V, off):
+    """Batches of fewer rows than CUs with unbounded windows: whole rows in
+    one workgroup (k64_kernel) while the windows fit its patch table (3/4 of its
+    slots), split rows from the first call whose windows may not, whole rows
+    again once the history is cleared; greedy, top-k and full-sort rows together
+    in the larger batches; ids, n, totals and candidates against the oracle
+    (sampler.nim:59-121)."""
+    rng = np.random.default_rng(V + B)
+    plist = []
+    for b in range(B):
+        k = [40, 64, 1, 0][b % 4] if B > 4 else 40
+        plist.append(dict(temperature=0.0 if b % 4 == 2 and B > 4 else 0.8, topK=k, topP=0.95, minP=0.05,
+                          repeatPenalty=1.1, repeatLastN=0, presencePenalty=0.2, frequencyPenalty=0.1, seed=b))
+    biases = [{int(i): float(rng.choice([-math.inf, 2.0])) for i in rng.choice(V, size=7, replace=False)}
+              for _ in range(B)]
+    flat = torch.zeros(B * V + off, dtype=torch.float32, device="cuda")
+    d = flat[off:].view(B, V)
+    s = pkg.BatchSampler([to_pkg_params(pkg, plist[b], biases[b]) for b in range(B)], V)
+    try:
+        hists = [[] for _ in range(B)]
+        seen = set()
+        for step, n in enumerate((40, 700, 2300, 18, 30, 3000)):
+            if step == 5:
+                s.clear_history()
+                hists = [[] for _ in range(B)]
+                n = 64
+            h = rng.choice(V, size=(B, n)).astype(np.int64)
+            s.accept(h)
+            for b in range(B):
+                hists[b] += h[b].tolist()
+            x = (rng.standard_normal((B, V)) * 3).astype(np.float32)
+            d.copy_(torch.from_numpy(x))
+            u = rng.random(B)
+            plan = s.plan()[0]
+            say(f"[windows] B={B} V={V} len={len(hists[0])} k64={plan.k64} slices={plan.slices}")
+            seen.add(int(plan.k64))
+            if V <= 262144:
+                assert plan.k64 == (1 if plan.slices == 1 else 0)
+                if len(hists[0]) + 7 > 3072:
+                    assert not plan.k64
+            ids, dbg = s.sample(d, torch.from_numpy(u).cuda(), debug_cap=64)
+            torch.cuda.synchronize()
+            compare_rows(x, plist, hists, biases, u, ids.cpu().numpy(),
+                         {k: v.cpu().numpy() for k, v in dbg.items()}, f"windows {B} {V} {step}")
+        assert seen == ({0, 1} if V <= 262144 else {0})
+    finally:
+        s.close()
