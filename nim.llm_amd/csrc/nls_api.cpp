@@ -909,8 +909,17 @@ int nls_clear_history(nls_sampler* s) {
 namespace {
 // One nls_sample call; may_alloc = false for the no-allocation entry point
 // (which then leaves handed-on rows to the streaming kernel's last workgroup).
+// `step`: the end ids and done flags of a generation step, which a call served
+// by k64_kernel alone makes too (step->made).
+struct StepCall {
+  const int32_t* eog;
+  int32_t n_eog;
+  int32_t* done;
+  bool made;
+};
 int sample_impl(nls_sampler* s, const float* d_logits, const double* d_u, int32_t* d_out,
-                const nls_debug* dbg, bool may_alloc, const int32_t* d_done = nullptr) {
+                const nls_debug* dbg, bool may_alloc, StepCall* step = nullptr) {
+  const int32_t* d_done = step ? step->done : nullptr;
   if (!s || !d_logits || !d_out) return NLS_ERR_INVALID_ARGUMENT;
   if (dbg && dbg->cap < 0) return NLS_ERR_INVALID_ARGUMENT;
   DebugPtrs dp;
@@ -1100,6 +1109,14 @@ int sample_impl(nls_sampler* s, const float* d_logits, const double* d_u, int32_
     ga.n_fixed = s->n_full_list;
   }
   a.ga = ga;
+  if (step && lp.k64 && a.gen_inline) {
+    a.eog = step->eog;
+    a.n_eog = step->n_eog;
+    a.step_done = step->done;
+    a.step_hist = s->hist;
+    a.step_len = s->hist_len;
+    step->made = true;
+  }
   lp.vec4 = (s->V % 4 == 0) && ((reinterpret_cast<uintptr_t>(d_logits) & 15) == 0);
   hipEvent_t e0 = s->prof_start, e1 = s->prof_stop, g0 = s->prof_gstart, g1 = s->prof_gstop;
   s->prof_start = s->prof_stop = s->prof_gstart = s->prof_gstop = nullptr;
@@ -1135,9 +1152,11 @@ int nls_generate_step(nls_sampler* s, const float* d_logits, const double* d_u, 
   if (!s || !d_logits || !d_out || !d_done || n_eog < 0 || (n_eog > 0 && !d_eog)) return NLS_ERR_INVALID_ARGUMENT;
   int rc = s->ensure_history(-1, 1);
   if (rc) return rc;
-  rc = sample_impl(s, d_logits, d_u, d_out, nullptr, true, d_done);
+  StepCall step{d_eog, n_eog, d_done, false};
+  rc = sample_impl(s, d_logits, d_u, d_out, nullptr, true, &step);
   if (rc) return rc;
-  NLS_HIP(launch_generate_step(d_out, s->B, s->V, d_eog, n_eog, d_done, s->hist, s->hist_len, s->hcap, s->stream));
+  if (!step.made)
+    NLS_HIP(launch_generate_step(d_out, s->B, s->V, d_eog, n_eog, d_done, s->hist, s->hist_len, s->hcap, s->stream));
   // rows that finished (or had finished) append nothing: the host lengths
   // become upper bounds
   for (int b = 0; b < s->B; ++b) s->h_len[b] += 1;

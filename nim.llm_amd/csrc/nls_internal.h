@@ -286,6 +286,13 @@ struct StreamArgs {
   const int32_t* row_list;
   int n_list;
   GenericArgs ga;
+  // k64_kernel serving every row of one step of batched generation
+  // (generate_step_kernel's work, by the row's own workgroup); step_done null: none
+  const int32_t* eog;
+  int n_eog;
+  int32_t* step_done;
+  int32_t* step_hist;
+  int64_t* step_len;
 };
 
 

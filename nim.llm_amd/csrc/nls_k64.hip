@@ -164,6 +164,26 @@ __device__ __forceinline__ void chain64(float* buf, float init) {
   wave_lds_sync();  // the chain's values are in buf for every lane
 }
 
+// One row's step of batched generation (chat.nim:204-208), as
+// generate_step_kernel makes it in a launch of its own (about 4 us behind the
+// sampling kernel's 28 at 24 x 50001): an end-of-generation id finishes the row,
+// any other is accepted into its history ring.  One wave; eog_lane: end id
+// `lane`, requested before the tail.
+__device__ __forceinline__ void k64_step(const StreamArgs& a, int row, int64_t hlen, int tok, int eog_lane) {
+  const int lane = lane_id();
+  bool end = __ballot(lane < a.n_eog && eog_lane == tok) != 0ull;
+  for (int j = kWave + lane; __ballot(j < a.n_eog) && !end; j += kWave)
+    end = __ballot(j < a.n_eog && a.eog[j] == tok) != 0ull;
+  if (lane != 0) return;
+  if (end) {
+    a.step_done[row] = 1;
+  } else {
+    const int slot = hlen < (int64_t{1} << 31) ? (int)((uint32_t)hlen % (uint32_t)a.hcap) : (int)(hlen % a.hcap);
+    a.step_hist[(int64_t)row * a.hcap + slot] = tok < 0 || tok >= a.V ? -1 : tok;
+    a.step_len[row] = hlen + 1;
+  }
+}
+
 // The reference's tail on one wave: lane i holds candidate i of the k <= 64
 // members in descending (value, index) order (x: key << 32 | id; 0 past k).
 // Softmax (sampler.nim:98-100, :51-57), top-p (:103-108), min-p (:110-114)
@@ -171,8 +191,8 @@ __device__ __forceinline__ void chain64(float* buf, float init) {
 // the top-p running sum, the draw's subtractions) run as single-lane chains
 // over `buf` (64 floats).  Past k the terms are +0, which leave a sum
 // unchanged; the top-p running sum at n - 1 is also the reference's total.
-__device__ __forceinline__ void k64_tail(uint64_t x, int k, const RowParams& P, double u_lane0, int row,
-                                         int32_t* out, const DebugPtrs& dbg, float* buf) {
+__device__ __forceinline__ int k64_tail(uint64_t x, int k, const RowParams& P, double u_lane0, int row,
+                                        int32_t* out, const DebugPtrs& dbg, float* buf) {
   const int lane = lane_id();
   const bool valid = lane < k;
   const int id = (int)(uint32_t)x;
@@ -222,13 +242,14 @@ __device__ __forceinline__ void k64_tail(uint64_t x, int k, const RowParams& P, 
     if (dbg.cand_ids) dbg.cand_ids[(int64_t)row * dbg.cap + lane] = id;
     if (dbg.cand_probs) dbg.cand_probs[(int64_t)row * dbg.cap + lane] = p;
   }
+  return tok;
 }
 
 // RK: the kinds of streamed rows the instance serves (kK64RowsAny: greedy and
 // top-k, kK64RowsTopK, kK64RowsGreedy).  An instance for one kind compiles
 // only that kind's code, so neither kind's registers and branches weigh on
 // the other's.
-template <bool VEC, int RK>
+template <bool VEC, int RK, bool STEP>
 __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2))) void k64_kernel(const StreamArgs a) {
   extern __shared__ __align__(16) unsigned char lds[];
   __shared__ int smem[kNW + 4];
@@ -947,6 +968,7 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2))) void k
         if (a.dbg.total) a.dbg.total[row] = 0.0f;
         if (a.dbg.path) a.dbg.path[row] = 1;
       }
+      if constexpr (STEP) k64_step(a, row, hlen, (x0 != x0) ? 0 : ri, lane < a.n_eog ? a.eog[lane] : 0);
       return;
     }
     // Top-k rows.  The listed patched ids whose final value reaches the
@@ -1040,9 +1062,12 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2))) void k
       NLS_STAMP_VALUE(row, 14, s_t0);
       NLS_STAMP_VALUE(row, 15, g);
       NLS_STAMP(row, 8);
+      int eog_lane = 0;
+      if (STEP && lane < a.n_eog) eog_lane = a.eog[lane];
       double u = 0.0;
       if (lane == 0) u = take_uniform(a.d_u, u_in, st0, st1, a.rng, row);
-      k64_tail(x, kk, P, u, row, a.out, a.dbg, s_chain);
+      const int tok = k64_tail(x, kk, P, u, row, a.out, a.dbg, s_chain);
+      if constexpr (STEP) k64_step(a, row, hlen, tok, eog_lane);
       NLS_STAMP(row, 11);
       return;
     }
@@ -1079,47 +1104,60 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2))) void k
       uint32_t* dl = reinterpret_cast<uint32_t*>(lds);
       generic_rows<kNT>(a.ga, 0, 1, count, whist, dl, dl + 256, smem, &s_u, reinterpret_cast<int*>(dl + 512),
                         s_rv, s_ri);
+      if constexpr (STEP) {  // those rows' steps
+        __syncthreads();
+        for (int i = wv; i < count; i += kNW) {
+          const int r = load_agent(&a.ga.generic_list[i]);
+          k64_step(a, r, a.hist_len[r], a.out[r], lane < a.n_eog ? a.eog[lane] : 0);
+        }
+      }
     }
   }
 }
 
-template <bool VEC>
+template <bool VEC, bool STEP>
 static void launch_k64_rows(const StreamArgs& a, const LaunchPlan& p, hipStream_t s) {
   const dim3 grid(a.row_list ? a.n_list : a.B);
   switch (p.k64_rows) {
     case kK64RowsTopK:
-      hipLaunchKernelGGL((k64_kernel<VEC, kK64RowsTopK>), grid, dim3(kNT), p.lds, s, a);
+      hipLaunchKernelGGL((k64_kernel<VEC, kK64RowsTopK, STEP>), grid, dim3(kNT), p.lds, s, a);
       break;
     case kK64RowsGreedy:
-      hipLaunchKernelGGL((k64_kernel<VEC, kK64RowsGreedy>), grid, dim3(kNT), p.lds, s, a);
+      hipLaunchKernelGGL((k64_kernel<VEC, kK64RowsGreedy, STEP>), grid, dim3(kNT), p.lds, s, a);
       break;
     default:
-      hipLaunchKernelGGL((k64_kernel<VEC, kK64RowsAny>), grid, dim3(kNT), p.lds, s, a);
+      hipLaunchKernelGGL((k64_kernel<VEC, kK64RowsAny, STEP>), grid, dim3(kNT), p.lds, s, a);
   }
 }
 
+// (The step's instances are apart: its code costs the others registers, 0.2 us
+// of 256 x 128256's 35.)
 hipError_t launch_k64(const StreamArgs& a, const LaunchPlan& p, hipStream_t s) {
-  if (p.vec4)
-    launch_k64_rows<true>(a, p, s);
+  if (a.step_done)
+    p.vec4 ? launch_k64_rows<true, true>(a, p, s) : launch_k64_rows<false, true>(a, p, s);
   else
-    launch_k64_rows<false>(a, p, s);
+    p.vec4 ? launch_k64_rows<true, false>(a, p, s) : launch_k64_rows<false, false>(a, p, s);
   return hipGetLastError();
 }
 
-template <bool VEC, int RK>
+template <bool VEC, bool STEP>
 static hipError_t set_k64_attr() {
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(&k64_kernel<VEC, RK>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)kK64MaxDynLds);
+  const void* kernels[] = {reinterpret_cast<const void*>(&k64_kernel<VEC, kK64RowsAny, STEP>),
+                           reinterpret_cast<const void*>(&k64_kernel<VEC, kK64RowsTopK, STEP>),
+                           reinterpret_cast<const void*>(&k64_kernel<VEC, kK64RowsGreedy, STEP>)};
+  for (const void* k : kernels) {
+    const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kK64MaxDynLds);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 hipError_t set_k64_attributes() {
   hipError_t e;
-  if ((e = set_k64_attr<true, kK64RowsAny>()) != hipSuccess) return e;
-  if ((e = set_k64_attr<true, kK64RowsTopK>()) != hipSuccess) return e;
-  if ((e = set_k64_attr<true, kK64RowsGreedy>()) != hipSuccess) return e;
-  if ((e = set_k64_attr<false, kK64RowsAny>()) != hipSuccess) return e;
-  if ((e = set_k64_attr<false, kK64RowsTopK>()) != hipSuccess) return e;
-  return set_k64_attr<false, kK64RowsGreedy>();
+  if ((e = set_k64_attr<true, false>()) != hipSuccess) return e;
+  if ((e = set_k64_attr<false, false>()) != hipSuccess) return e;
+  if ((e = set_k64_attr<true, true>()) != hipSuccess) return e;
+  return set_k64_attr<false, true>();
 }
 
 }  // namespace nls

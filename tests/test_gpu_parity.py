@@ -1682,3 +1682,54 @@ def test_windows_that_outgrow_the_patch_table(pkg, torch, B, V, off):
         assert seen == ({0, 1} if V <= 262144 else {0})
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("kind,B,V", [("topk", 7, 50001), ("greedy", 20, 50000), ("both", 260, 8192), ("topk", 3, 131072)])
+def test_generate_step_in_the_sampling_kernel(pkg, torch, kind, B, V):
+    """Batches k64_kernel serves alone make the step in its workgroups
+    (chat.nim:204-208): rows that finish or accept there, rows handed on to its
+    last workgroup (ascending logits: every candidate buffer overflows), rings
+    that wrap, and more end ids than a wave has lanes."""
+    rng = np.random.default_rng(B + V)
+    steps = 7
+    eog = [int(i) for i in rng.choice(V, size=70, replace=False)]
+    plist = []
+    for b in range(B):
+        greedy = kind == "greedy" or (kind == "both" and b % 3 == 0)
+        plist.append(dict(temperature=0.0 if greedy else 0.8, topK=int(rng.choice([5, 40, 64])), topP=0.95, minP=0.0,
+                          repeatPenalty=1.3, repeatLastN=3 if b % 2 else 0, presencePenalty=0.5, frequencyPenalty=0.2,
+                          seed=b + 1))
+    streams = [list(O.uniforms(plist[b]["seed"], steps)) for b in range(B)]
+    hist, done, used = [[] for _ in range(B)], [False] * B, [0] * B
+    say(f"[step_in_kernel] {kind} B={B} V={V}")
+    s = pkg.BatchSampler([to_pkg_params(pkg, p, {}) for p in plist], V)
+    d_done = torch.zeros(B, dtype=torch.int32, device="cuda")
+    d_eog = torch.tensor(eog, dtype=torch.int32, device="cuda")
+    try:
+        plan = s.plan()[0]
+        assert plan.k64 and not plan.generic_launch
+        for t in range(steps):
+            x = (rng.standard_normal((B, V)) * 2.0).astype(np.float32)
+            x[1] = np.sort(x[1])
+            x[2 % B] = np.linspace(-8, 8, V, dtype=np.float32)
+            if t >= 2:
+                x[rng.integers(3, B) if B > 3 else 2, eog[-1 - t]] += 30.0
+            out = s.generate_step(torch.from_numpy(x).cuda(), d_eog, d_done).cpu().numpy()
+            for b in range(B):
+                if done[b]:
+                    assert out[b] == -1, (t, b)
+                    continue
+                u = 0.0
+                if plist[b]["temperature"] > 0:
+                    u = streams[b][used[b]]
+                    used[b] += 1
+                res, _, _, _ = oracle_row(x[b], plist[b], hist[b], {}, u, O.EXPF_CR)
+                assert out[b] == res.id, (t, b, int(out[b]), res.id)
+                if res.id in eog:
+                    done[b] = True
+                else:
+                    hist[b].append(res.id)
+            assert [bool(v) for v in d_done.cpu().numpy()] == done, t
+        assert any(done) and not all(done)
+    finally:
+        s.close()
