@@ -7,13 +7,13 @@
 // bound by the requests one CU keeps in flight; the exponentials: by float64
 // issue; the sum: by the latency of its windows), and fewer rows than CUs
 // leave the rest of the chip idle.  Here the launches are:
-//   A. split_max_kernel: each slice's maximum m and an estimate a of
-//      sum exp(l - m) (v_exp_f32), one read of the row.
+//   A. split_max_kernel: the maximum m of each 1024 logits (a wave's) and an
+//      estimate a of their sum exp(l - m) (v_exp_f32), one read of the row.
 //   B. split_terms_kernel: mx = the largest m.  The reference's index-order
 //      fp32 sum s of exp(l - mx) is a scan of parity maps (nls_seqsum.h) once
 //      the running sum's binade is known, so each group of 256 terms takes
-//      the binade of its estimated running sum (the a of the slices below,
-//      this slice's own terms) and stores its map for that binade.
+//      the binade of its estimated running sum (the a of the waves' logits
+//      below, this wave's own terms) and stores its map for that binade.
 //      A term's part of a map is round(e / u), u the binade's spacing.  An
 //      fp32 estimate y of e (|y - e| <= kSplitErr e) settles it unless y / u
 //      lies within kSplitErr y / u of a half; only those terms (about 1 in
@@ -145,7 +145,8 @@ __device__ __forceinline__ int unpack_code(uint64_t u) { return (int)((u >> 52) 
 
 struct RowWork {  // one row's part of the workspace
   uint64_t* maps;   // [ns * 16] (nll: the slices' float64 sums)
-  float2* part;     // [ns]: m and a of each slice
+  float2* part;     // [np]: m and a of each wave's 1024 logits
+  int np;
   SplitRowInfo* info;
   float* gmax;      // [ns * 16], topTokens: maxima of 256 logits each
   uint64_t* list;   // [kSplitList], topTokens: key << 32 | index
@@ -153,7 +154,8 @@ struct RowWork {  // one row's part of the workspace
 __device__ __forceinline__ RowWork row_work(const SplitArgs& a, int row) {
   RowWork w;
   w.maps = a.maps + (int64_t)row * a.ns * kSplitGroups;
-  w.part = a.part + (int64_t)row * a.ns;
+  w.np = a.ns * kWpb;
+  w.part = a.part + (int64_t)row * w.np;
   w.info = a.info + row;
   w.gmax = a.gmax + (int64_t)row * a.ns * kSplitGroups;
   w.list = a.list + (int64_t)row * kSplitList;
@@ -269,7 +271,6 @@ __device__ __forceinline__ float replay_group(float s, const float (&e)[4], int 
 
 template <int KIND>
 __global__ __launch_bounds__(kNT) void split_max_kernel(SplitArgs a) {
-  __shared__ float s_m[kWpb], s_a[kWpb];
   const int row = (int)(blockIdx.x / (unsigned)a.ns), sl = (int)(blockIdx.x % (unsigned)a.ns);
   const int tid = (int)threadIdx.x, lane = lane_id(), wv = wave_id();
   const float* x = a.logits + (int64_t)row * a.V;
@@ -299,19 +300,8 @@ __global__ __launch_bounds__(kNT) void split_max_kernel(SplitArgs a) {
       t = __ballot(nan) ? __builtin_nanf("") : 0.0f;
     }
   }
-  if (lane == 0) {
-    s_m[wv] = m;
-    s_a[wv] = t;  // (a NaN or +inf logit leaves a NaN)
-  }
-  __syncthreads();
-  if (tid == 0) {
-    float mm = s_m[0], t2 = 0.0f;
-    for (int k = 1; k < kWpb; ++k) mm = __builtin_fmaxf(mm, s_m[k]);
-    if (KIND != kSplitNll)
-      for (int k = 0; k < kWpb; ++k)
-        t2 += s_m[k] > -__builtin_inff() ? s_a[k] * __builtin_amdgcn_exp2f((s_m[k] - mm) * kLog2e) : s_a[k];
-    w.part[sl] = make_float2(mm, t2);
-  }
+  // (a NaN or +inf logit leaves a NaN in t)
+  if (lane == 0) w.part[sl * kWpb + wv] = make_float2(m, t);
 }
 
 // ---------------------------------------------------------------- launch B
@@ -321,7 +311,6 @@ __global__ __launch_bounds__(kNT) void split_max_kernel(SplitArgs a) {
 template <int KIND>
 __global__ __launch_bounds__(kNT, 8) void split_terms_kernel(SplitArgs a) {
   __shared__ double s_pow2[kExpfPow2Count];
-  __shared__ float s_tot[kWpb];
   const int row = (int)(blockIdx.x / (unsigned)a.ns), sl = (int)(blockIdx.x % (unsigned)a.ns);
   const int tid = (int)threadIdx.x, lane = lane_id(), wv = wave_id();
   const float* x = a.logits + (int64_t)row * a.V;
@@ -330,19 +319,26 @@ __global__ __launch_bounds__(kNT, 8) void split_terms_kernel(SplitArgs a) {
   const int g0 = sl * kSplitGroups + wv * kGpw;  // this wave's first group
   f32x4 v[kGpw];
   load_groups(x, g0 * kGroup, n, v);
-  if (tid < kExpfPow2Count) s_pow2[tid] = kExpfPow2J64[tid];
-  // the row's maximum, and the estimated sum of the slices below this one
-  float mx = -__builtin_inff(), pre = 0.0f, unused;
-  if (a.ns <= kWave) {
-    const float2 p = lane < a.ns ? w.part[lane] : make_float2(mx, 0.0f);
-    mx = wave_max_f(p.x, unused);
-    if (lane < sl) pre = p.y * __builtin_amdgcn_exp2f((p.x - mx) * kLog2e);
+  // (every wave writes the whole table, the same values: no barrier, so the
+  // workgroup's waves run on their own)
+  s_pow2[lane] = kExpfPow2J64[lane];
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  // the row's maximum, and the estimated sum of the waves' logits below this one's
+  const int me = sl * kWpb + wv;
+  float mx = -__builtin_inff(), P = 0.0f, unused;
+  if (w.np <= 2 * kWave) {
+    const float2 none = make_float2(mx, 0.0f);
+    const float2 p0 = lane < w.np ? w.part[lane] : none;
+    const float2 p1 = lane + kWave < w.np ? w.part[lane + kWave] : none;
+    mx = wave_max_f(__builtin_fmaxf(p0.x, p1.x), unused);
+    if (lane < me) P = p0.y * __builtin_amdgcn_exp2f((p0.x - mx) * kLog2e);
+    if (lane + kWave < me) P += p1.y * __builtin_amdgcn_exp2f((p1.x - mx) * kLog2e);
   } else {
-    for (int i = lane; i < a.ns; i += kWave) mx = __builtin_fmaxf(mx, w.part[i].x);
+    for (int i = lane; i < w.np; i += kWave) mx = __builtin_fmaxf(mx, w.part[i].x);
     mx = wave_max_f(mx, unused);
-    for (int i = lane; i < sl; i += kWave) pre += w.part[i].y * __builtin_amdgcn_exp2f((w.part[i].x - mx) * kLog2e);
+    for (int i = lane; i < me; i += kWave) P += w.part[i].y * __builtin_amdgcn_exp2f((w.part[i].x - mx) * kLog2e);
   }
-  pre = wave_sum_f(pre);
+  P = wave_sum_f(P);
   if (KIND == kSplitTop) {
     // The list's bound.  The row's 256-element maxima, merged to 64: the m-th
     // largest of those is a logit that m distinct elements reach.  It is
@@ -379,10 +375,6 @@ __global__ __launch_bounds__(kNT, 8) void split_terms_kernel(SplitArgs a) {
     gsum[g] = (y[g][0] + y[g][1]) + (y[g][2] + y[g][3]);
   }
   wave_sum4(gsum);
-  if (lane == 0) s_tot[wv] = (gsum[0] + gsum[1]) + (gsum[2] + gsum[3]);
-  __syncthreads();
-  float P = pre;
-  for (int k = 0; k < wv; ++k) P += s_tot[k];
   const int ng = (n + kGroup - 1) / kGroup;
   int E[kGpw];
   float inc[kGpw];        // the group's increment, as far as it is settled
@@ -471,7 +463,7 @@ __global__ __launch_bounds__(kNT) void split_nll_kernel(SplitArgs a) {
   load_groups(x, i0 - 4 * lane, n, v);
   if (tid < kExp64Table) s_t[tid] = exp64_table_entry(tid);
   float mx = -__builtin_inff(), unused;
-  for (int i = lane; i < a.ns; i += kWave) mx = __builtin_fmaxf(mx, w.part[i].x);
+  for (int i = lane; i < w.np; i += kWave) mx = __builtin_fmaxf(mx, w.part[i].x);
   mx = wave_max_f(mx, unused);
   __syncthreads();
   double ps = 0.0;
@@ -502,10 +494,8 @@ __global__ __launch_bounds__(kWave) void split_nll_sum_kernel(SplitArgs a) {
   const float lt = t >= 0 && t < a.V ? a.logits[(int64_t)row * a.V + t] : __builtin_nanf("");
   float mx = -__builtin_inff(), unused;
   double s = 0.0;
-  for (int i = lane; i < a.ns; i += kWave) {
-    mx = __builtin_fmaxf(mx, w.part[i].x);
-    s += __longlong_as_double((long long)w.maps[i]);
-  }
+  for (int i = lane; i < w.np; i += kWave) mx = __builtin_fmaxf(mx, w.part[i].x);
+  for (int i = lane; i < a.ns; i += kWave) s += __longlong_as_double((long long)w.maps[i]);
   mx = wave_max_f(mx, unused);
   for (int o = kWave / 2; o > 0; o >>= 1) s += __shfl_xor(s, o);
   if (lane == 0) a.logp[row] = -((double)(lt - mx) - log(s));
@@ -678,7 +668,7 @@ __global__ __launch_bounds__(kWalkNT) void split_walk_kernel(SplitArgs a) {
   float s = 0.0f;
   if (tid < kExpfPow2Count) sh.pow2[tid] = kExpfPow2J64[tid];
   float mx = -__builtin_inff(), bad = 0.0f, unused;
-  for (int i = lane; i < a.ns; i += kWave) {
+  for (int i = lane; i < w.np; i += kWave) {
     mx = __builtin_fmaxf(mx, w.part[i].x);
     bad += w.part[i].y;  // (a sum of finite estimates is no NaN)
   }
@@ -840,7 +830,7 @@ size_t split_workspace(int kind, int64_t rows, int64_t V, int m) {
   if (kind == kSplitNll && (V < kSplitMinNllV || rows > kSplitMaxNllRows)) return 0;
   // the list's bound is the m-th largest of up to 64 maxima of 256 logits
   if (kind == kSplitTop && m > std::min<int64_t>(kWave, V / kGroup)) return 0;
-  size_t b = (size_t)rows * sizeof(SplitRowInfo) + (size_t)(rows * ns) * (kSplitGroups * 8 + 8);
+  size_t b = (size_t)rows * sizeof(SplitRowInfo) + (size_t)(rows * ns) * (kSplitGroups * 8 + kWpb * 8);
   if (kind == kSplitTop) b += (size_t)(rows * ns) * kSplitGroups * 4 + (size_t)rows * kSplitList * 8;
   return b;
 }
@@ -854,7 +844,7 @@ hipError_t launch_split(int kind, SplitArgs a, int rows, void* work, hipStream_t
   a.maps = reinterpret_cast<uint64_t*>(p);
   p += (size_t)slices * kSplitGroups * 8;
   a.part = reinterpret_cast<float2*>(p);
-  p += (size_t)slices * 8;
+  p += (size_t)slices * kWpb * 8;
   a.list = reinterpret_cast<uint64_t*>(p);  // (topTokens only)
   p += (size_t)rows * kSplitList * 8;
   a.gmax = reinterpret_cast<float*>(p);
