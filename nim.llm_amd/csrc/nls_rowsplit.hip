@@ -17,7 +17,7 @@
 //      A term's part of a map is round(e / u), u the binade's spacing.  An
 //      fp32 estimate y of e (|y - e| <= kSplitErr e) settles it unless y / u
 //      lies within kSplitErr y / u of a half; only those terms (about 1 in
-//      8,000) take the correctly rounded exponential, whose float64
+//      16,000) take the correctly rounded exponential, whose float64
 //      arithmetic bounded the one-launch kernels' sum.
 //   C. split_walk_kernel: a workgroup per row walks the maps with the exact
 //      sum.  A group's map is used when its binade is the sum's and the sum
@@ -31,10 +31,10 @@
 // walk in its last slice (agent-scope fences, or write-through stores and a
 // wait) cost 30 us of 256 x 128256's 95 us in launch B.
 // Measured, one pass, one launch -> split: topTokens, n = 5, 32 x 128256 147 -> 40 us;
-// softmax 256 x 128256 186 -> 158, 1 x 128256 147 -> 30; logProb 201 x 50001 66 -> 45,
+// softmax 256 x 128256 186 -> 158, 1 x 128256 147 -> 30; logProb 201 x 50001 66 -> 44,
 // 1 x 50001 59 -> 25; perplexity's term 8 x 128256 37 -> 10.  Of softmax's 158 us: A 20,
-// B 59 (516 vector instructions a wave, 28 us at full issue; the rest is
-// latency), C 20 (latency of one wave), D 51 (262 MB at 5.1 TB/s).
+// B 57 (about 500 vector instructions a wave, 28 us at full issue), C 20 (latency
+// of one wave), D 51 (262 MB at 5.1 TB/s).
 #include "nls_device.h"
 #include "nls_exp64.h"
 #include "nls_rowsplit.h"
@@ -828,6 +828,12 @@ size_t split_workspace(int kind, int64_t rows, int64_t V, int m) {
   // 160 rows 46 -> 41, 256 rows 55 -> 60; V = 32000: 8 rows 11.6 -> 10.4, 96 rows
   // 12.1 -> 14.0)
   if (kind == kSplitNll && (V < kSplitMinNllV || rows > kSplitMaxNllRows)) return 0;
+  // softmax's fourth launch pays from longer rows on, or from more rows than
+  // CUs (the one launch's second round): 8 x 9000 27.4 -> 29.6 us, 160 x 12288 35.5 ->
+  // 34.8, 256 x 12288 36.0 -> 36.6, 256 x 14000 41.6 -> 40.4, 400 x 8192 55 -> 44.  logProb and
+  // topTokens gain from kSplitMinV on (256 x 9000 27.6 -> 27.2, 1 x 8192 23 -> 17; 42 -> 30,
+  // 38 -> 20)
+  if (kind == kSplitSoftmax && rows <= 256 && V < (rows <= 192 ? 12288 : 14336)) return 0;
   // the list's bound is the m-th largest of up to 64 maxima of 256 logits
   if (kind == kSplitTop && m > std::min<int64_t>(kWave, V / kGroup)) return 0;
   size_t b = (size_t)rows * sizeof(SplitRowInfo) + (size_t)(rows * ns) * (kSplitGroups * 8 + kWpb * 8);

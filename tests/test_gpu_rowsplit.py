@@ -63,7 +63,7 @@ def _rows(V, seed):
 
 # below the split, its first size, ragged sizes, whole and nearly whole slices,
 # real vocabularies, the last size of the split and the first past it
-SIZES = [8191, 8192, 8193, 12287, 12289, 50001, 128256, 151936, 1 << 20, (1 << 20) + 1]
+SIZES = [8191, 8192, 8193, 12287, 12288, 12289, 50001, 128256, 151936, 1 << 20, (1 << 20) + 1]
 
 
 @pytest.mark.parametrize("V", SIZES)
@@ -158,10 +158,14 @@ def test_workspace_rule(pkg):
     """A short, odd or missing workspace runs the one-launch kernels; the
     sizes the split covers ask for one."""
     L = pkg.lib()
-    assert L.nls_rows_workspace(0, 4, 8191, 0) == 0
-    assert L.nls_rows_workspace(0, 4, 8192, 0) > 0
+    assert L.nls_rows_workspace(1, 4, 8191, 0) == 0
+    assert L.nls_rows_workspace(1, 4, 8192, 0) > 0
+    assert [L.nls_rows_workspace(0, r, v, 0) > 0 for r, v in
+            [(4, 12287), (4, 12288), (193, 12288), (256, 14336), (257, 8192)]] == [False, True, False, True, True]
+    assert [L.nls_rows_workspace(3, r, v, 0) > 0 for r, v in
+            [(4, 40959), (4, 40960), (160, 50000), (161, 50000)]] == [False, True, True, False]
     assert L.nls_rows_workspace(2, 4, 8192, 33) == 0
-    assert L.nls_rows_workspace(2, 4, 8192, 32) > L.nls_rows_workspace(0, 4, 8192, 0)
+    assert L.nls_rows_workspace(2, 4, 8192, 32) > L.nls_rows_workspace(1, 4, 8192, 0)
     assert L.nls_rows_workspace(0, 0, 8192, 0) == 0
     assert L.nls_rows_workspace(0, 1, (1 << 20) + 1, 0) == 0
     assert L.nls_rows_workspace(9, 1, 50000, 0) == 0
