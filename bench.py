@@ -322,7 +322,7 @@ def bench_top_tokens(args):
            "config": {"workload": f"{args.workload} logits, topTokens n={n}", "B": B, "V": V},
            "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": achieved / HBM_PEAK_GBS, "traffic": None,
-                        "kernel": "top_tokens_kernel", "kernel_avg_us": ms * 1e3,
+                        "kernel": "split_max + split_terms + split_walk + top_tokens_kernel", "kernel_avg_us": ms * 1e3,
                         "algorithmic_bytes_per_launch": nbytes,
                         "single_lane_sum_chain_us": chain_us},
            "parity_spot_check": {"rows": 3, "bit_exact": ok}}
@@ -465,7 +465,8 @@ def bench_softmax(args, logp):
     nbytes = float(B * V * 4 + (B * V * 4 if not logp else B * 16))
     achieved = nbytes / (ms * 1e-3) / 1e9
     name = "logProb terms" if logp else "softmaxInPlace rows"
-    kern = "softmax_kernel<true>" if logp else "softmax_kernel<false>"
+    # (rows split over workgroups: the launches of one call together)
+    kern = "split_max + split_terms + split_walk" + ("" if logp else " + split_out")
     res = {"metric": f"{name} (rows/sec) at B={B} x V={V} fp32", "value": B / (ms * 1e-3),
            "unit": "rows/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
            "ms_per_step": ms, "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
@@ -554,11 +555,11 @@ def bench_lm_head(args):
     achieved = nbytes / (ms * 1e-3) / 1e9
     path = "int8 activations" if O.matmul_uses_act(t, cols, nb, args.lm_exact) else "dequantise + dotF32"
     if path != "int8 activations":
-        kern = "lm_float_kernel"
+        kern = "lm_half_kernel" if args.lm_type in ("F16", "BF16") else "lm_float_kernel"
     elif nb == 1 and (cols // 32 + 63) // 64 <= 4:
         kern = "lm_int1_kernel (activations quantised in the kernel)"
     else:
-        kern = "quant_act_kernel + lm_int_kernel"
+        kern = "quant_act_kernel + " + ("lm_batch_kernel" if args.lm_type.endswith("_K") else "lm_int_kernel")
     res = {"metric": f"LM head calls/sec ({rows} x {cols} {args.lm_type}, nb={nb})",
            "value": 1e3 / ms, "unit": "calls/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
            "ms_per_step": ms, "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
