@@ -656,6 +656,35 @@ __device__ __forceinline__ float walk_round(float s, int c0, int nev, const floa
   return seq_ldexp((float)S, E - 23);
 }
 
+// The sum of a row with a NaN term (one wave): the reference's adds leave the first
+// NaN term as it is from there on, sign and payload included.  topTokens orders
+// the quotients by them: with another NaN than the row's own as the sum, the
+// entries that are NaN themselves would leave their places among the others.
+__device__ __forceinline__ float first_nan_term(const RowWork& w, const float* x, int n, float mx) {
+  const int lane = lane_id();
+  int i0 = 0;  // (no finite logit: -inf - -inf is the first term)
+  if (mx > -__builtin_inff()) {
+    for (int k = 0; k < w.np; k += kWave) {  // the first 1024 logits whose estimate is a NaN
+      const float y = k + lane < w.np ? w.part[k + lane].y : 0.0f;
+      const uint64_t hit = __ballot(y != y);
+      if (hit) {
+        i0 = (k + __ffsll((unsigned long long)hit) - 1) * kGpw * kGroup;
+        break;
+      }
+    }
+  }
+  for (int i = i0; i < n; i += kWave) {
+    const float d = i + lane < n ? x[i + lane] - mx : 0.0f;
+    const uint64_t hit = __ballot(d != d);
+    if (hit) {
+      const int l = __ffsll((unsigned long long)hit) - 1;
+      const float t = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(d), l));
+      return t + t;  // (the exponential's NaN)
+    }
+  }
+  return __builtin_nanf("");
+}
+
 template <bool LOGP>
 __global__ __launch_bounds__(kWalkNT) void split_walk_kernel(SplitArgs a) {
   __shared__ __align__(16) WalkShared sh;
@@ -751,8 +780,8 @@ __global__ __launch_bounds__(kWalkNT) void split_walk_kernel(SplitArgs a) {
       if (wv == 0) s = walk_round(c0 == kHeadGroups ? sh.head_sum : s, c0, nev, x, n, mx, sh);
       __syncthreads();  // (the round's LDS is free again)
     }
-  } else {
-    s = __builtin_nanf("");
+  } else if (wv == 0) {
+    s = first_nan_term(w, x, n, mx);
   }
   if (tid == 0) {
     if (LOGP) {

@@ -123,6 +123,60 @@ def test_split_rows(pkg, torch, V):
                 assert np.array_equal(pr[i], want[order[:m]]), (V, off, name, n)
 
 
+@pytest.mark.parametrize("V", [12288, 50001, 131072])
+def test_nan_rows_as_in_one_launch(pkg, torch, V):
+    """Rows with NaN or infinite logits, NaNs of any sign and payload: every
+    output is the one-launch kernels', bit for bit (topTokens orders NaN
+    probabilities by their bits, so the sum's own NaN decides its ids)."""
+    rng = np.random.default_rng(V + 9)
+    nans = np.array([0x7FC00000, 0xFFC00000, 0x7FC00123, 0xFFC00123, 0x7F800001, 0xFF800007], np.uint32)
+    rows = []
+    for i in range(18):
+        x = rng.standard_normal(V).astype(np.float32)
+        k = [1, 2, 60, 400][i % 4]
+        x.view(np.uint32)[rng.choice(V, k, replace=False)] = nans[i % 6] if i < 6 else rng.choice(nans, k)
+        if i % 5 == 4:
+            x[rng.integers(0, V, size=3)] = np.inf
+        rows.append(x)
+    for at in (0, 1023, 1024, V - 1):  # the edges of the 1024 logits a wave sums
+        x = rng.standard_normal(V).astype(np.float32)
+        x.view(np.uint32)[at] = 0xFFC00123
+        rows.append(x)
+    x = rng.standard_normal(V).astype(np.float32)
+    x[V // 2] = np.inf
+    rows.append(x)
+    x = np.full(V, -np.inf, np.float32)
+    x.view(np.uint32)[V // 2] = 0x7FC00123
+    rows += [x, np.full(V, -np.inf, np.float32), np.full(V, np.inf, np.float32)]
+    R = len(rows)
+    say(f"[rowsplit] NaN rows V={V}, {R} rows")
+    d = torch.from_numpy(np.stack(rows)).cuda()
+    t = torch.from_numpy(rng.integers(0, V, size=R).astype(np.int32)).cuda()
+    vp = ctypes.c_void_p
+    L = pkg.lib()
+
+    def p(q):
+        return vp(q.data_ptr())
+
+    sm = torch.empty(R, V, device="cuda")
+    pkg.check(L.nls_softmax_rows(p(d), R, V, p(sm), None), "one launch")
+    prob = torch.empty(R, device="cuda")
+    logp = torch.empty(R, dtype=torch.float64, device="cuda")
+    pkg.check(L.nls_log_prob(p(d), R, V, p(t), p(prob), p(logp), None), "one launch")
+    got = pkg.log_prob_device(d, t)
+    for g, w in ((pkg.softmax_device(d), sm), (got[0], prob)):
+        bad = (g.view(torch.int32) != w.view(torch.int32)).reshape(R, -1).any(1).nonzero().reshape(-1).tolist()
+        assert not bad, (V, bad)
+    assert torch.equal(got[1].view(torch.int64), logp.view(torch.int64))
+    for n in (1, 5, 48):
+        ids = torch.empty(R, n, dtype=torch.int32, device="cuda")
+        pr = torch.empty(R, n, device="cuda")
+        pkg.check(L.nls_top_tokens(p(d), R, V, n, p(ids), p(pr), None), "one launch")
+        gi, gp = pkg.top_tokens_device(d, n)
+        assert torch.equal(gi, ids), (V, n, (gi != ids).any(1).nonzero().reshape(-1).tolist())
+        assert torch.equal(gp.view(torch.int32), pr.view(torch.int32)), (V, n)
+
+
 def test_split_in_a_graph(pkg, torch):
     """The split calls captured once and replayed on changing logits, with
     eager calls between the replays."""
