@@ -102,6 +102,61 @@ __device__ __forceinline__ bool tie_members(uint64_t* mem, int ge, int gt, int k
   return (int)__popcll(mk) == k;
 }
 
+// The same for ties past the 64 largest: `ent` holds the n <= kK64RankCap
+// candidates in any order; the k members go to mem[0..k).  Every count reads the
+// list again: the path is rare, and values kept in registers would spill those of
+// the row's common path.  (Rows with more than 64 entries at or above T went to
+// the whole-row path, which the grid's last workgroup runs for one row after
+// another: 128 x 128256, k = 40, logits in steps of 1/4, 7.6 ms a call; 42 us here.)
+__device__ __forceinline__ bool tie_members_list(const uint64_t* ent, int n, uint64_t* mem, int k, uint32_t T,
+                                                 int ibits) {
+  const int lane = lane_id();
+  // entries with lo <= key << 32 | index <= hi
+  auto count = [&](uint64_t lo, uint64_t hi) {
+    int c = 0;
+#pragma unroll 1
+    for (int i = lane; i - lane < n; i += kWave) {
+      const uint64_t x = i < n ? ent[i] : 0ull;
+      c += (int)__popcll(__ballot(i < n && x >= lo && x <= hi));
+    }
+    return c;
+  };
+  const uint64_t t = (uint64_t)T << 32;
+  // p*: the smallest r with at least k entries of index <= r
+  uint32_t r = 0u;
+#pragma unroll 1
+  for (int b = ibits - 1; b >= 0; --b) {
+    const uint32_t c = r | ((1u << b) - 1u);
+    int below = 0;
+#pragma unroll 1
+    for (int i = lane; i - lane < n; i += kWave) {
+      const uint64_t x = i < n ? ent[i] : 0ull;
+      below += (int)__popcll(__ballot(i < n && x >= t && (uint32_t)x <= c));
+    }
+    if (below < k) r |= 1u << b;
+  }
+  // the m-th largest tie index up to p*
+  const int m = k - count(t + 0x100000000ull, ~0ull);
+  uint32_t q = 0u;
+#pragma unroll 1
+  for (int b = ibits - 1; b >= 0; --b) {
+    const uint32_t c = q | (1u << b);
+    if (c <= r && count(t | c, t | r) >= m) q = c;
+  }
+  int base = 0;
+#pragma unroll 1
+  for (int i = lane; i - lane < n; i += kWave) {
+    const uint64_t x = i < n ? ent[i] : 0ull;
+    const bool in = i < n && ((uint32_t)(x >> 32) > T || (x >= (t | q) && x <= (t | r)));
+    const uint64_t mk = __ballot(in);
+    const int at = base + (int)__popcll(mk & lanes_below());
+    if (in && at < k) mem[at] = x;
+    base += (int)__popcll(mk);
+  }
+  wave_lds_sync();
+  return base == k;
+}
+
 // Descending rank sort of n <= 64 distinct 64-bit entries mem[0..n) (LDS,
 // 16-byte aligned; what lies past n is ignored): every lane counts the entries
 // above its own, reading them two at a time, then the entries move to their
@@ -1043,9 +1098,13 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2))) void k
         const uint32_t kx = (uint32_t)(x >> 32);
         const int ge = (int)__popcll(__ballot(lane < nl && kx >= T));
         const int gt = (int)__popcll(__ballot(lane < nl && kx > T));
-        // all entries >= T must lie within the 64 ranks held
+        // all entries >= T must lie within the 64 ranks held, else the whole
+        // list is looked at again
         if (ge == nl && N > nl) {
-          rovf = true;
+          if (tie_members_list(cand, N, s_flist, kk, T, 32 - __clz(len > 1 ? len - 1 : 1)))
+            x = rank_sort64(s_flist, kk);
+          else
+            rovf = true;
         } else if (tie_members(s_flist, ge, gt, kk, T, 32 - __clz(len > 1 ? len - 1 : 1))) {
           x = rank_sort64(s_flist, kk);
         } else {

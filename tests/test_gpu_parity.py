@@ -1733,3 +1733,30 @@ def test_generate_step_in_the_sampling_kernel(pkg, torch, kind, B, V):
         assert any(done) and not all(done)
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("B,V,k", [(12, 50001, 40), (9, 128256, 64), (12, 32000, 1), (12, 32000, 64), (270, 8192, 40)])
+def test_ties_past_the_ranks_held(pkg, torch, B, V, k):
+    """Equal values at the k-th place around the 64 entries the last wave holds
+    and the 256 the workgroup ranks: the heap rule's members and the whole tail
+    (sampler.nim:85-121) against the oracle, made by the streaming kernel
+    itself (path 2: no row is handed on)."""
+    rng = np.random.default_rng(V + k)
+    say(f"[ties] B={B} V={V} k={k}")
+    x = np.minimum(rng.standard_normal((B, V)), 3.0).astype(np.float32)
+    counts = [2, 23, 24, 25, 43, 44, 63, 64, 65, 255, 256, 257, 900, 1700]
+    plist = []
+    for b in range(B):
+        gt = [0, k // 2, k - 1][b % 3]
+        m = counts[(b * 5 + b // 14) % len(counts)]
+        at = rng.choice(V, size=gt + m, replace=False)
+        x[b, at[:gt]] = 9.0 + rng.integers(1, 4, size=gt).astype(np.float32) / 4
+        x[b, at[gt:]] = 9.0
+        plist.append(dict(temperature=0.9, topK=k, topP=0.97, minP=0.0, repeatPenalty=1.2 if b % 2 else 1.0, repeatLastN=8,
+                          presencePenalty=0.0, frequencyPenalty=0.0, seed=b))
+    hist = rng.integers(0, V, size=(B, 8)).astype(np.int64)
+    u = rng.random(B)
+    params = [to_pkg_params(pkg, p, {}) for p in plist]
+    ids, dbg = run_gpu(pkg, torch, x, params, hist, u, debug_cap=64)
+    assert (dbg["path"] == 2).all(), np.flatnonzero(dbg["path"] != 2)[:8]
+    compare_rows(x, plist, [list(h) for h in hist], [{}] * B, u, ids, dbg, f"ties {B} {V} {k}")
