@@ -348,17 +348,31 @@ struct Geometry {
 // Whether a batch of fewer rows than CUs still streams each row in one
 // workgroup.  k64_kernel's one workgroup has no candidates to exchange, and
 // its serial phases are shorter: sampled at k = 40, 1 x 128256 29 us against 38 split,
-// 24 x 50001 27.5 against 30.6, 200 x 128256 32 against 97, 1 x 262144 46 against 53.  A
-// greedy row has nothing to exchange but its maximum, so few long ones are
-// split (1 x 128256: 14.3 against 15.7, 8 x 200000: 17.8 against 19.5; 64 x 128256: 33
-// against 16).  Past 262144 ids the bitmap leaves too little LDS to the patch
-// table; k > 64 streams whole rows at a workgroup's pace and stays split.
-// (Small batches of greedy beside top-k rows and no full sorts, `both`, also
-// stay: their split plan is the one the tests of NaN rows over slices expect.)
-bool whole_rows(int B, int64_t V, int kmax, int ncu, bool both) {
+// 24 x 50001 27.5 against 30.6, 200 x 128256 32 against 97, 1 x 262144 46 against 53.
+// Where the split rows stay:
+// - few rows of more than 200,000 ids with little to exchange (1 x 262144: k = 1 28
+//   against 26, k = 5 30.1 against 29.3);
+// - greedy rows alone, which exchange nothing but their maximum: fewer than 48, or
+//   80 of more than 200,000 ids (24 x 50001 with 256 windowed ids 23 against 20,
+//   24 x 128256 of mostly -inf 31 against 25, 64 x 262144 of those 47 against 41; 48 x
+//   128256 22 against 33, of mostly -inf 31 against 33; 48 x 50001 19 against 23, with
+//   one half -inf 22 against 20), but for 16 or more short ones, whose generation
+//   step then needs no launch of its own;
+// - greedy beside top-k rows, whose kernel serves both kinds: below 16 rows
+//   (8 x 65536 31 against 30, 12 x 128256 32 against 37: even), and shorter rows below
+//   48 (24 x 65536 32 against 30, 48 x 65536 32 against 34; 16 x 98304 31 against 33);
+//   beside full sorts, which take the whole-row path's time in either plan, they
+//   do not count;
+// - past 262144 ids, where the bitmap leaves too little LDS to the patch table;
+//   k > 64, which streams whole rows at a workgroup's pace.
+bool whole_rows(int B, int64_t V, int kmax, int ncu, bool greedy, bool full) {
   if (B >= ncu || V <= kSmallRowV) return true;
-  if (kmax > kWaveTopK || V > kWholeRowV || both) return false;
-  return kmax > 0 || V <= kWholeGreedyV || B >= kWholeGreedyRows;
+  if (kmax > kWaveTopK || V > kWholeRowV) return false;
+  if (kmax == 0)
+    return greedy && (B >= (V > kWholeFewKV ? kWholeGreedyRows : kWholeMixedRows) ||
+                      (B >= kWholeFewRows && V <= kWholeGreedyV));
+  if (greedy && !full) return B >= (V >= kWholeLongV ? kWholeFewRows : kWholeMixedRows);
+  return kmax >= 8 || B >= 8 || V <= kWholeFewKV;
 }
 
 Geometry plan_geometry(int B, int64_t V, int kmax, int ncu, int max_patch, bool whole) {
@@ -579,20 +593,16 @@ int nls_create(const nls_params* per_row, int32_t batch, int64_t vocab, void* st
   if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1)
     ncu = 256;
   int kfast = kmax;
-  bool both = false;
-  {
-    bool greedy = false, topk = false, full = false;
-    for (int b = 0; b < B; ++b) {
-      const RowParams& r = s->h_rp[b];
-      greedy |= r.mode == kModeGreedy;
-      (r.mode == kModeTopK && r.k <= kMaxTopKFast ? topk : full) |= r.mode != kModeGreedy;
-    }
-    both = greedy && topk && !full;
+  bool greedy = false, full = false;  // (full: rows of the whole-row path)
+  for (int b = 0; b < B; ++b) {
+    const RowParams& r = s->h_rp[b];
+    greedy |= r.mode == kModeGreedy;
+    full |= r.mode == kModeFull || (r.mode == kModeTopK && r.k > kMaxTopKFast);
   }
-  Geometry g = plan_geometry(B, vocab, kfast, ncu, max_patch, whole_rows(B, vocab, kfast, ncu, both));
+  Geometry g = plan_geometry(B, vocab, kfast, ncu, max_patch, whole_rows(B, vocab, kfast, ncu, greedy, full));
   while (kfast > 0 && (g.lds > max_dynamic_lds() || (g.nt != 512 && g.pcap < 256))) {
     kfast = kfast * 7 / 8;
-    g = plan_geometry(B, vocab, kfast, ncu, max_patch, whole_rows(B, vocab, kfast, ncu, both));
+    g = plan_geometry(B, vocab, kfast, ncu, max_patch, whole_rows(B, vocab, kfast, ncu, greedy, full));
   }
   // (false only for vocabularies far beyond 2^19; the slice's byte size must
   // also fit the 32-bit range of the kernel's buffer loads)

@@ -52,9 +52,12 @@ constexpr int kWaveCap = 256;        // per-wave candidate buffer of the k <= 64
 constexpr int kWaveTopK = 64;        // largest k of the wave path
 constexpr size_t kDualStreamLds = 68 * 1024;  // dynamic LDS of a 512-thread workgroup, two per CU
 constexpr int64_t kSmallRowV = 49152;  // rows up to this size stream in one workgroup
-constexpr int64_t kWholeRowV = 262144;    // and, with k <= 64, rows up to this (whole_rows)
-constexpr int64_t kWholeGreedyV = 98304;  // greedy rows alone: up to this, or in batches from
-constexpr int kWholeGreedyRows = 16;      // this many
+constexpr int64_t kWholeRowV = 262144;   // and, with k <= 64, rows up to this; the lines
+constexpr int kWholeGreedyRows = 80;     // of whole_rows (nls_api.cpp)
+constexpr int64_t kWholeGreedyV = 53248;
+constexpr int kWholeFewRows = 16, kWholeMixedRows = 48;
+constexpr int64_t kWholeLongV = 81920;
+constexpr int64_t kWholeFewKV = 200000;
 
 // k64_kernel (greedy and top-k <= 64 rows, one 1024-thread workgroup per
 // row): LDS = patch bitmap | hash table (4 words per slot) | per-wave

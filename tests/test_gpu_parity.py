@@ -1760,3 +1760,57 @@ def test_ties_past_the_ranks_held(pkg, torch, B, V, k):
     ids, dbg = run_gpu(pkg, torch, x, params, hist, u, debug_cap=64)
     assert (dbg["path"] == 2).all(), np.flatnonzero(dbg["path"] != 2)[:8]
     compare_rows(x, plist, [list(h) for h in hist], [{}] * B, u, ids, dbg, f"ties {B} {V} {k}")
+
+
+def _kinds_params(kinds, b, **kw):
+    d = dict(temperature=0.8, topK=40, topP=0.95, minP=0.0, repeatPenalty=1.1, repeatLastN=16, presencePenalty=0.0,
+             frequencyPenalty=0.0, seed=b + 1)
+    d.update({"greedy": dict(temperature=0.0, topK=0), "topk": {}, "topk2": dict(topK=2),
+              "full": dict(topK=0)}[kinds[b % len(kinds)]])
+    d.update(kw)
+    return d
+
+
+# (kinds of rows, batch, vocabulary, whole rows?): both sides of every line
+WHOLE_LINES = [
+    (["topk"], 1, 49216, 1), (["topk"], 1, 262144, 1), (["topk"], 1, 262208, 0), (["topk"], 200, 128256, 1),
+    (["topk2"], 7, 200064, 0), (["topk2"], 8, 200064, 1), (["topk2"], 7, 200000, 1),
+    (["greedy"], 15, 53248, 0), (["greedy"], 16, 53248, 1), (["greedy"], 47, 53312, 0), (["greedy"], 48, 53312, 1),
+    (["greedy"], 12, 98304, 0), (["greedy"], 48, 200000, 1), (["greedy"], 79, 200064, 0), (["greedy"], 80, 200064, 1),
+    (["greedy", "topk"], 15, 128256, 0), (["greedy", "topk", "topk", "topk"], 16, 128256, 1),
+    (["greedy", "topk"], 16, 81920, 1), (["greedy", "topk"], 47, 81856, 0), (["greedy", "topk"], 48, 50001, 1),
+    (["topk", "topk", "topk", "greedy"], 64, 128256, 1), (["greedy", "topk", "full"], 9, 65536, 1),
+]
+
+
+def test_whole_row_lines(pkg, torch):
+    """Which batches of fewer rows than CUs run whole rows in one workgroup
+    each and which are split, on both sides of every line of the rule."""
+    for kinds, B, V, whole in WHOLE_LINES:
+        s = pkg.BatchSampler([to_pkg_params(pkg, _kinds_params(kinds, b), {}) for b in range(B)], V)
+        try:
+            plan = s.plan()[0]
+            assert (plan.k64, plan.slices == 1) == (whole, bool(whole)), (kinds, B, V, plan.k64, plan.slices)
+        finally:
+            s.close()
+
+
+@pytest.mark.parametrize("B,V", [(18, 98304), (49, 50001), (16, 128256), (15, 128256), (30, 65536)])
+def test_greedy_beside_topk_rows(pkg, torch, B, V):
+    """Greedy and top-k rows in one batch of fewer rows than CUs, on whole rows and
+    split: ids, candidates and totals against the oracle (sampler.nim:59-121),
+    and on whole rows the generation step (chat.nim:204-208) too."""
+    rng = np.random.default_rng(B * V)
+    say(f"[greedy_beside_topk] B={B} V={V}")
+    kinds = ["greedy", "topk", "topk", "topk2"]
+    plist = [_kinds_params(kinds, b) for b in range(B)]
+    biases = [{int(i): float(rng.choice([-math.inf, 2.0])) for i in rng.choice(V, size=5, replace=False)} for _ in range(B)]
+    x = (rng.standard_normal((B, V)) * 2.5).astype(np.float32)
+    x[2] = np.round(x[2] * 2) / 2
+    x[4, ::2] = -np.inf
+    hist = rng.integers(0, V, size=(B, 20)).astype(np.int64)
+    u = rng.random(B)
+    ids, dbg = run_gpu(pkg, torch, x, [to_pkg_params(pkg, p, biases[b]) for b, p in enumerate(plist)], hist, u, debug_cap=64)
+    compare_rows(x, plist, [list(h) for h in hist], biases, u, ids, dbg, f"greedy beside topk {B} {V}")
+    if B >= (16 if V >= 81920 else 48):
+        test_generate_step_in_the_sampling_kernel(pkg, torch, "both", B, V)
