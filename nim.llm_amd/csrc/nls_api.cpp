@@ -143,6 +143,8 @@ struct nls_sampler {
   std::vector<int64_t> h_len;     // accepted ids per row (an upper bound while !len_exact)
   bool len_exact = true;          // false after nls_accept_device, whose rows may skip
   std::vector<int> need_window;   // repeat_last_n (>0) or -1 (whole history), 0 if unused
+  std::vector<int> h_rise;        // biases that may raise a logit
+  std::vector<char> h_win_rise;   // penalties that may raise one
   int hcap = 0;
 
   // streaming-kernel plan
@@ -158,8 +160,10 @@ struct nls_sampler {
   // counters it would have handed on are cleared before the next call
   bool counters_dirty = false;
   int hbits = 0;   // k64_kernel's hash table: 2^hbits slots
-  // Fewer rows than CUs with windows that may outgrow that table: the split
-  // rows' plan, for the calls whose windows may have (S > 1: there is one).
+  // Fewer rows than CUs with more patched ids than whole rows take well
+  // (whole_patches): the split rows' plan, for the calls whose windows may hold
+  // so many (S > 1: there is one).
+  int64_t whole_cap = 0;
   struct SplitPlan {
     int S = 1, L = 0, xcd_map = 0, ccap = 0, nwords = 0, pcap = 0, mcap = 0, kcap = 0, offA = 0, pc = 0, nt = 0, q = 0;
     size_t lds = 0;
@@ -260,19 +264,26 @@ struct nls_sampler {
   // handed on to the whole-row path, which then gets a launch of its own
   // across the CUs rather than the streaming kernel's last workgroup.
   int64_t k64_patches() const { return (int64_t)((1 << hbits) - (1 << hbits) / 4); }
-  bool split_now() const { return alt.S > 1 && windows_exceed(k64_patches()); }
+  bool split_now() const { return alt.S > 1 && (windows_exceed(whole_cap) || risers_exceed(kK64PListCap)); }
   bool window_may_overflow() const {
     return windows_exceed(split_now() ? alt.pcap : plan.k64 ? k64_patches() : (int64_t)pcap);
   }
   bool windows_exceed(int64_t cap) const {
     for (int b = 0; b < B; ++b) {
       const RowParams& r = h_rp[b];
-      if (!r.fast) continue;
-      int64_t w = 0;
-      if (need_window[b] != 0) w = need_window[b] > 0 ? std::min<int64_t>(need_window[b], h_len[b]) : h_len[b];
-      if (w + r.bias_cnt > cap) return true;
+      if (r.fast && window(b) + r.bias_cnt > cap) return true;
     }
     return false;
+  }
+  // The same for the patched ids whose final value may be above the logit: k64_kernel
+  // lists each of them, wherever its row's candidates lie.
+  bool risers_exceed(int64_t cap) const {
+    for (int b = 0; b < B; ++b)
+      if (h_rp[b].fast && (h_win_rise[b] ? window(b) : 0) + h_rise[b] > cap) return true;
+    return false;
+  }
+  int64_t window(int b) const {
+    return need_window[b] == 0 ? 0 : need_window[b] > 0 ? std::min<int64_t>(need_window[b], h_len[b]) : h_len[b];
   }
 
   // Grows the history ring so that every row's window fits after `extra`
@@ -349,6 +360,8 @@ struct Geometry {
 // workgroup.  k64_kernel's one workgroup has no candidates to exchange, and
 // its serial phases are shorter: sampled at k = 40, 1 x 128256 29 us against 38 split,
 // 24 x 50001 27.5 against 30.6, 200 x 128256 32 against 97, 1 x 262144 46 against 53.
+// (Rows in ascending order, where no threshold keeps anything out, are the
+// exception: 8 x 128256 90 against 43, 24 x 50001 49 against 42, 200 x 50001 51 against 88.)
 // Where the split rows stay:
 // - few rows of more than 200,000 ids with little to exchange (1 x 262144: k = 1 28
 //   against 26, k = 5 30.1 against 29.3);
@@ -373,6 +386,22 @@ bool whole_rows(int B, int64_t V, int kmax, int ncu, bool greedy, bool full) {
                       (B >= kWholeFewRows && V <= kWholeGreedyV));
   if (greedy && !full) return B >= (V >= kWholeLongV ? kWholeFewRows : kWholeMixedRows);
   return kmax >= 8 || B >= 8 || V <= kWholeFewKV;
+}
+
+// The patched ids (window and biases) up to which such a batch's calls run
+// whole rows: one workgroup builds the table that the slices of a split row
+// share out, and a greedy row meets most of its patched ids above some lane's
+// best, so it lists them.  Sampled at k = 40 with windows of 3/8, 1/2 and 3/4 of the
+// table's slots, whole against split: 24 x 50001 32, 36 and 50 us against 34, 35 and 38;
+// 24 x 128256 35, 41 and 55 against 45, 45 and 49; 128 x 50001 33, 37 and 52 against 44, 44
+// and 49; 200 x 50001 33, 37 and 58 against 69, 70 and 82.  Greedy, windows of 512 and
+// 1024: 80 x 50001 27 and 32 against 28 and 28; 24 x 50001, windows of 64 and 256: 17 and 23
+// against 19 and 20.  Greedy beside top-k, a window of 1024: 48 x 50001 34 against 36.
+// (Past the table itself a row takes the whole-row path, milliseconds.)
+int64_t whole_patches(int B, int64_t V, int slots, bool greedy, bool topk) {
+  if (greedy) return topk ? 1024 : B >= kWholeGreedyRows ? 512 : B >= kWholeMixedRows ? 256 : 128;
+  if (B >= kWholeManyRows) return slots / 4 * 3;
+  return B >= 64 || V >= kWholeLongV ? slots / 2 : slots / 8 * 3;
 }
 
 Geometry plan_geometry(int B, int64_t V, int kmax, int ncu, int max_patch, bool whole) {
@@ -515,6 +544,8 @@ int nls_create(const nls_params* per_row, int32_t batch, int64_t vocab, void* st
   s->h_rp.resize(B);
   s->h_len.assign(B, 0);
   s->need_window.assign(B, 0);
+  s->h_rise.assign(B, 0);
+  s->h_win_rise.assign(B, 0);
 
   // bias tables: per row, in-range ids, last value wins, sorted by id
   std::vector<int32_t> bid;
@@ -563,6 +594,8 @@ int nls_create(const nls_params* per_row, int32_t batch, int64_t vocab, void* st
       r.mode = k < vocab ? kModeTopK : kModeFull;
       if (r.mode == kModeTopK && k <= kMaxTopKFast) kmax = std::max(kmax, (int)k);
     }
+    for (int j = 0; j < r.bias_cnt; ++j) s->h_rise[b] += !(bval[(size_t)r.bias_off + j] <= 0.0f);
+    s->h_win_rise[b] = (r.rp_active && !(r.rp32 >= 1.0f)) || !(r.freq >= 0.0) || !(r.pres >= 0.0);
     if (r.pen_active) s->need_window[b] = p.repeat_last_n > 0 ? (int)std::min<int64_t>(p.repeat_last_n, 1 << 24) : -1;
     if (max_patch >= 0) {
       if (r.pen_active && p.repeat_last_n <= 0)
@@ -649,10 +682,11 @@ int nls_create(const nls_params* per_row, int32_t batch, int64_t vocab, void* st
         any_topk |= s->h_rp[b].mode == kModeTopK;
       }
       if (any_greedy != any_topk) s->plan.k64_rows = any_greedy ? kK64RowsGreedy : kK64RowsTopK;
-      // the split rows' plan beside it where a window may outgrow the table
-      // (a row past it takes the whole-row path, milliseconds; the slices of a
-      // split row hold a table each)
-      if (B < ncu && vocab > kSmallRowV && (max_patch < 0 || max_patch > s->k64_patches())) {
+      // the split rows' plan beside it where the patched ids may be more than
+      // whole rows take well (the slices of a split row hold a table each)
+      s->whole_cap = whole_patches(B, vocab, 1 << hb, any_greedy, any_topk);
+      if (B < ncu && vocab > kSmallRowV &&
+          (max_patch < 0 || max_patch > std::min<int64_t>(s->whole_cap, kK64PListCap))) {
         const Geometry d = plan_geometry(B, vocab, kfast, ncu, max_patch, false);
         if (d.S > 1 && d.wave && d.nt == 256 && d.lds <= max_dynamic_lds() && d.pcap >= 256) {
           auto& t = s->alt;

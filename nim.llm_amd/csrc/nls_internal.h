@@ -52,10 +52,10 @@ constexpr int kWaveCap = 256;        // per-wave candidate buffer of the k <= 64
 constexpr int kWaveTopK = 64;        // largest k of the wave path
 constexpr size_t kDualStreamLds = 68 * 1024;  // dynamic LDS of a 512-thread workgroup, two per CU
 constexpr int64_t kSmallRowV = 49152;  // rows up to this size stream in one workgroup
-constexpr int64_t kWholeRowV = 262144;   // and, with k <= 64, rows up to this; the lines
-constexpr int kWholeGreedyRows = 80;     // of whole_rows (nls_api.cpp)
+constexpr int64_t kWholeRowV = 262144;   // and, with k <= 64, rows up to this; the lines of
+constexpr int kWholeGreedyRows = 80;     // whole_rows and whole_patches (nls_api.cpp)
 constexpr int64_t kWholeGreedyV = 53248;
-constexpr int kWholeFewRows = 16, kWholeMixedRows = 48;
+constexpr int kWholeFewRows = 16, kWholeMixedRows = 48, kWholeManyRows = 192;
 constexpr int64_t kWholeLongV = 81920;
 constexpr int64_t kWholeFewKV = 200000;
 

@@ -1814,3 +1814,39 @@ def test_greedy_beside_topk_rows(pkg, torch, B, V):
     compare_rows(x, plist, [list(h) for h in hist], biases, u, ids, dbg, f"greedy beside topk {B} {V}")
     if B >= (16 if V >= 81920 else 48):
         test_generate_step_in_the_sampling_kernel(pkg, torch, "both", B, V)
+
+
+@pytest.mark.parametrize("kind,B,V,window,bias,whole", [
+    ("topk", 5, 50001, 1500, 0, 1), ("topk", 5, 50001, 1600, 0, 0), ("topk", 3, 131072, 2040, 0, 1),
+    ("topk", 3, 131072, 2060, 0, 0), ("topk", 3, 131072, 0, 1000, 1), ("topk", 9, 65536, 10, 1500, 0),
+    ("topk", 4, 200000, 1030, 0, 0), ("greedy", 20, 50000, 120, 0, 1), ("greedy", 20, 50000, 140, 0, 0),
+    ("greedy", 50, 57344, 300, 0, 0), ("raised", 4, 128256, 1030, 0, 0),
+])
+def test_many_patched_ids_on_split_rows(pkg, torch, kind, B, V, window, bias, whole):
+    """Fewer rows than CUs with more windowed or biased ids than whole rows take
+    well run split, so no row is handed on for them: the plan on both sides of
+    each line, and the rows against the oracle (sampler.nim:59-121)."""
+    rng = np.random.default_rng(V + window + bias)
+    say(f"[many_patched] {kind} B={B} V={V} window={window} bias={bias}")
+    plist, biases = [], []
+    for b in range(B):
+        plist.append(dict(temperature=0.0 if kind == "greedy" else 0.8, topK=40, topP=0.95, minP=0.0,
+                          repeatPenalty=0.9 if kind == "raised" else 1.1, repeatLastN=0, presencePenalty=0.1,
+                          frequencyPenalty=0.0, seed=b))
+        ids = rng.choice(V, size=bias, replace=False) if bias else []
+        biases.append({int(i): float(v) for i, v in zip(ids, rng.uniform(0.5, 2.0, size=bias))})
+    x = (rng.standard_normal((B, V)) * 2.5).astype(np.float32)
+    hist = np.stack([rng.choice(V, size=window, replace=False) for _ in range(B)]).astype(np.int64)
+    u = rng.random(B)
+    s = pkg.BatchSampler([to_pkg_params(pkg, p, q) for p, q in zip(plist, biases)], V)
+    try:
+        if window:
+            s.accept(hist)
+        plan = s.plan()[0]
+        assert plan.k64 == whole and (plan.slices == 1) == bool(whole)
+        ids, dbg = s.sample(torch.from_numpy(x).cuda(), torch.from_numpy(u).cuda(), debug_cap=64)
+        ids, dbg = ids.cpu().numpy(), {k: v.cpu().numpy() for k, v in dbg.items()}
+    finally:
+        s.close()
+    assert (dbg["path"] <= 2).all(), dbg["path"]
+    compare_rows(x, plist, [list(h) for h in hist], biases, u, ids, dbg, f"many patched {kind} {B} {V}")
