@@ -441,16 +441,16 @@ struct IntArgs {
   float* y;
 };
 
-// The 32-weight formats past lm_int1_kernel's reach (Q4_0 with more than four
-// hidden states, long rows).  One wave per group of `rw` rows.  For each row
-// the wave's lanes form the integer sums of their blocks (64 blocks = 2048
-// weights per pass) and write the blocks' fp32 terms to LDS.  Then one lane
-// per row adds its row's terms in block order.  Up to kLmNBC activation rows
-// share each load of a block.
+// Past lm_int1_kernel's reach (Q4_0 with more than four hidden states, long
+// rows) where lm_batch_kernel does not win (int_kernel_wins).  One wave per
+// group of `rw` rows.  For each row the wave's lanes form the integer partials
+// of their slices (64 slices = 2048 weights per pass), the 8 lanes of a K
+// format's block add theirs, and the block's last lane writes the block's fp32
+// term to LDS.  Then one lane per row adds its row's terms in block order.  Up
+// to kLmNBC activation rows share each load of a weight slice.
 template <int T>
 __global__ __launch_bounds__(kLmNT) void lm_int_kernel(IntArgs a) {
   using F = Fmt<T>;
-  static_assert(F::LPB == 1, "one lane per block");
   extern __shared__ float s_term[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int64_t row0 = ((int64_t)blockIdx.x * (kLmNT / 64) + wave) * a.rw;
@@ -463,15 +463,21 @@ __global__ __launch_bounds__(kLmNT) void lm_int_kernel(IntArgs a) {
     for (int rr = 0; rr < nrow; ++rr) {
       const uint8_t* rp = a.w + (row0 + rr) * a.row_bytes;
       for (int pass = 0; pass < a.passes; ++pass) {
-        const int ib = pass * 64 + lane;
-        if (ib >= a.nblk) continue;
-        const typename F::Wt w = F::load_w(rp + (int64_t)ib * F::TS, 0);
+        const int s = pass * 64 + lane;
+        const int ib = s / F::LPB, p = s % F::LPB;
+        if (ib >= a.nblk) continue;  // (a K format's block: all of its 8 lanes)
+        const typename F::Wt w = F::load_w(rp + (int64_t)ib * F::TS, p);
         for (int bb = 0; bb < nbc; ++bb) {
           const int64_t brow = b0 + bb;
-          const typename F::Act act = load_act<T>(a.aqs + brow * a.cols + (int64_t)ib * F::BL, 0);
+          const typename F::Act act = load_act<T>(a.aqs + brow * a.cols + (int64_t)ib * F::BL, p);
           int si, sm;
-          F::partial(w, act, 0, si, sm);
-          term[(bb * a.rw + rr) * a.nblk + ib] = F::term(w, si, sm, a.ad[brow * a.nblk + ib]);
+          F::partial(w, act, p, si, sm);
+          if (F::LPB == 8) {
+            si = group8_sum(si);
+            if (F::HAS_MIN) sm = group8_sum(sm);
+          }
+          if (p == F::LPB - 1)
+            term[(bb * a.rw + rr) * a.nblk + ib] = F::term(w, si, sm, a.ad[brow * a.nblk + ib]);
         }
       }
     }
@@ -1095,8 +1101,46 @@ hipError_t launch_int1(const LmHeadCall& c, int nblk, hipStream_t s) {
   return hipGetLastError();
 }
 
+// lm_int_kernel's rows per wave: 16, fewer when the per-wave term buffer would pass 4 KiB
+int int_rows_per_wave(int nblk, int nb) {
+  const int nbc = std::min(nb, kLmNBC);
+  int rw = 16;
+  while (rw > 1 && (int64_t)nbc * rw * nblk * 4 > 4096) rw >>= 1;
+  return rw;
+}
+
+// Whether lm_int_kernel takes a K format's rows sooner than lm_batch_kernel.
+// The latter walks a row's blocks one after another, whatever the states, at
+// about `block_us` each as long as the row tiles fill no more than the chip;
+// the former splits a row over its lanes, but starts again for every four
+// states.  So it wins for few states of long rows, and the fewer rows the more
+// (us, lm_int_kernel / lm_batch_kernel, 1 state): Q6_K 4000 x 16384 105 / 204, 32000 x
+// 14336 186 / 165; 2 states: Q4_K 2000 x 16384 64 / 86, 32000 x 16384 168 / 107; Q6_K
+// 4000 x 8192 64 / 89, 32000 x 8192 112 / 94; 5 states: Q6_K 8000 x 8192 102 / 90.  Both
+// estimates are fits to 800 such pairs (256 to 128256 rows of 1024 to 28672 columns,
+// 1 to 64 states), within a few per cent where the two lie close.
+bool int_kernel_wins(int type, int64_t rows, int64_t cols, int nb, int64_t row_bytes) {
+  const int nblk = (int)(cols / 256);
+  const double block_us = type == 12 ? 1.3 : type == 13 ? 1.9 : nblk <= 32 ? 2.7 : 2.9;
+  const int64_t groups = ((nb + 31) / 32 + 3) / 4;
+  const double tiles = (double)((rows + 127) / 128 * groups);
+  // (a term buffer past 64 KB of LDS is not lm_int_kernel's either)
+  const int64_t buffer = (int64_t)(kLmNT / 64) * std::min(nb, kLmNBC) * int_rows_per_wave(nblk, nb) * nblk * 4;
+  if (buffer > 65536) return false;
+  const double batch = nblk * block_us * std::max(1.0, 0.5 + tiles / (2 * device_cus()));
+  const double units = (double)int_rows_per_wave(nblk, nb) * (double)((cols / 32 + 63) / 64);
+  double rows_us = 0.0;
+  for (int left = nb; left > 0 && rows_us < batch; left -= kLmNBC) {
+    const int k = std::min(left, kLmNBC);
+    const double wave = units * (0.3 + 0.31 * k);
+    const double all = (double)rows * (double)row_bytes / 2.6e6 + (double)rows * (double)cols * k * 1e-8;
+    rows_us += std::max(wave, all) + 0.4 * std::min(wave, all);
+  }
+  return rows_us < batch;
+}
+
 template <int T>
-hipError_t launch_int32(const LmHeadCall& c, int nblk, int passes, hipStream_t s) {
+hipError_t launch_int_rows(const LmHeadCall& c, int nblk, int passes, hipStream_t s) {
   IntArgs a;
   a.w = static_cast<const uint8_t*>(c.w);
   a.rows = c.rows;
@@ -1108,13 +1152,9 @@ hipError_t launch_int32(const LmHeadCall& c, int nblk, int passes, hipStream_t s
   a.nblk = nblk;
   a.passes = passes;
   a.y = c.y;
-  const int nbc = std::min(c.nb, kLmNBC);
-  // rows per wave: 16, fewer when the per-wave term buffer would pass 4 KiB
-  int rw = 16;
-  while (rw > 1 && (int64_t)nbc * rw * a.nblk * 4 > 4096) rw >>= 1;
-  a.rw = rw;
-  const size_t lds = (size_t)(kLmNT / 64) * nbc * rw * a.nblk * sizeof(float);
-  const int64_t grid = (c.rows + (int64_t)rw * (kLmNT / 64) - 1) / ((int64_t)rw * (kLmNT / 64));
+  a.rw = int_rows_per_wave(nblk, c.nb);
+  const size_t lds = (size_t)(kLmNT / 64) * std::min(c.nb, kLmNBC) * a.rw * a.nblk * sizeof(float);
+  const int64_t grid = (c.rows + (int64_t)a.rw * (kLmNT / 64) - 1) / ((int64_t)a.rw * (kLmNT / 64));
   hipLaunchKernelGGL(lm_int_kernel<T>, dim3((unsigned)grid), dim3(kLmNT), lds, s, a);
   return hipGetLastError();
 }
@@ -1138,8 +1178,9 @@ hipError_t launch_int(const LmHeadCall& c, hipStream_t s) {
   hipLaunchKernelGGL(quant_act_kernel<F::BL>, dim3((unsigned)qgrid), dim3(kLmNT), 0, s, c.x, n, c.act_qs, c.act_d);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  if constexpr (F::LPB == 8) return launch_lm_batch(c, s);
-  else return launch_int32<T>(c, nblk, passes, s);
+  if constexpr (F::LPB == 8)
+    if (!int_kernel_wins(T, c.rows, c.cols, c.nb, c.row_bytes)) return launch_lm_batch(c, s);
+  return launch_int_rows<T>(c, nblk, passes, s);
 }
 
 template <int T, int P, int NB>

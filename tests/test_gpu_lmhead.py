@@ -254,6 +254,21 @@ def test_batched_states_parity(pkg, name):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("name", ["Q4_K", "Q5_K", "Q6_K"])
+def test_few_states_of_long_rows_parity(pkg, name):
+    """K formats past one lane's registers, on both sides of the line between
+    the lanes' kernel (few states of long rows) and the matrix cores: row
+    counts around the rows a wave takes, whole and partial passes of 2048
+    weights, one to nine states: every logit bit for bit."""
+    t = TYPES[name]
+    for rows, nb, blocks in [(1, 1, 33), (63, 1, 64), (65, 1, 112), (257, 2, 36), (40, 2, 64), (33, 3, 63), (130, 3, 112),
+                             (17, 4, 65), (300, 4, 40), (31, 5, 112), (9, 8, 120), (70, 9, 112), (2500, 1, 34),
+                             (2048, 4, 9), (1000, 2, 17), (128, 6, 20)]:
+        print(f"lm_head few states {name} rows={rows} cols={256 * blocks} nb={nb}", flush=True)
+        run_case(pkg, t, rows, 256 * blocks, nb, seed=rows + nb)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("name", ["F16", "BF16"])
 def test_half_weights_parity(pkg, name):
     """Two-byte weights around the edges of their kernel: rows around a wave's
