@@ -1353,7 +1353,8 @@ int nls_set_rng_state(nls_sampler* s, int32_t row, uint64_t a0, uint64_t a1) {
 // the caller brought the bytes, else the one-launch kernels: the same results.
 static bool use_split(int kind, int64_t rows, int64_t vocab, int m, const void* work, size_t work_bytes) {
   const size_t need = nls::split_workspace(kind, rows, vocab, m);
-  return need > 0 && work && work_bytes >= need && (reinterpret_cast<uintptr_t>(work) & 15) == 0;
+  return need > 0 && work && work_bytes >= need && (reinterpret_cast<uintptr_t>(work) & 15) == 0 &&
+         nls::split_pays(kind, rows, vocab);
 }
 
 size_t nls_rows_workspace(int32_t op, int32_t rows, int64_t vocab, int32_t n) {

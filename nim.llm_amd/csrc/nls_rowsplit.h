@@ -49,6 +49,7 @@ struct SplitArgs {
 
 // Workspace bytes, 0 where the one-launch kernels run the call.
 size_t split_workspace(int kind, int64_t rows, int64_t V, int m);
+bool split_pays(int kind, int64_t rows, int64_t V);
 hipError_t launch_split(int kind, SplitArgs a, int rows, void* work, hipStream_t s);
 // topTokens' last launch (nls_kernels.hip).
 hipError_t launch_split_top(const SplitArgs& a, int rows, hipStream_t s);

@@ -26,13 +26,14 @@
 //      costs time, never a bit.  logProb ends here.
 //   D. softmax: exp(l - mx) / s for every element (split_out_kernel).
 //      topTokens: the entries B listed, in order (top_tokens_kernel<true>).
-//      perplexity: B sums float64 exponentials, C adds the slices' sums.
+//      perplexity: B sums float64 exponentials as row_nll_kernel's waves do, C
+//      adds the waves' sums.
 // The launches hand over through memory: an arrival count per row with the
 // walk in its last slice (agent-scope fences, or write-through stores and a
 // wait) cost 30 us of 256 x 128256's 95 us in launch B.
 // Measured, one pass, one launch -> split: topTokens, n = 5, 32 x 128256 147 -> 40 us;
 // softmax 256 x 128256 186 -> 158, 1 x 128256 147 -> 30; logProb 201 x 50001 66 -> 44,
-// 1 x 50001 59 -> 25; perplexity's term 8 x 128256 37 -> 10.  Of softmax's 158 us: A 20,
+// 1 x 50001 59 -> 25; perplexity's term 8 x 128256 36 -> 12.  Of softmax's 158 us: A 20,
 // B 57 (about 500 vector instructions a wave, 28 us at full issue), C 20 (latency
 // of one wave), D 51 (262 MB at 5.1 TB/s).
 #include "nls_device.h"
@@ -144,7 +145,7 @@ __device__ __forceinline__ SeqMap unpack_map(uint64_t u) {
 __device__ __forceinline__ int unpack_code(uint64_t u) { return (int)((u >> 52) & 0xff); }
 
 struct RowWork {  // one row's part of the workspace
-  uint64_t* maps;   // [ns * 16] (nll: the slices' float64 sums)
+  uint64_t* maps;   // [ns * 16] (nll: 16 float64 sums)
   float2* part;     // [np]: m and a of each wave's 1024 logits
   int np;
   SplitRowInfo* info;
@@ -448,57 +449,98 @@ __global__ __launch_bounds__(kNT, 8) void split_terms_kernel(SplitArgs a) {
   }
 }
 
-// perplexity's term (model.nim:578-583): the slice's part of the float64 sum
-// of exp(l - mx), a fixed tree over the threads.
-__global__ __launch_bounds__(kNT) void split_nll_kernel(SplitArgs a) {
+// perplexity's term (model.nim:578-583).  row_nll_kernel's 1024 threads each add
+// their own float64 exponentials in index order (a thread's are 1024 float4 groups
+// apart, or 1024 logits in rows off 16 bytes), then the waves' lanes in a tree, then
+// the 16 waves.  The same sum here, so that a position's term does not depend on
+// how many are scored together: a workgroup per row and one of those waves, whose
+// exponentials the workgroup's waves share out (64 slots of the 64 lanes per chunk,
+// through LDS) and its first wave adds in their order.  Bound by float64 issue
+// and, for few rows, by the chunks' barriers: 8 x 50001 9.6 us, 8 x 128256 11.6 (row_nll_kernel
+// 19.5 and 36.3; slices of 4096 logits with a tree of their own 9.9 and 9.9).  (Sixteen
+// waves, the last one adding a chunk behind the others: 10.2 and 12.3.)
+constexpr int kNllNT = 512;
+constexpr int kNllWaves = kNllNT / kWave;
+constexpr int kNllParts = 16;                      // row_nll_kernel's waves
+constexpr int kNllThreads = kNllParts * kWave;     // and threads
+constexpr int kNllSlots = 64;                      // of a chunk
+constexpr int kNllPer = kNllSlots / kNllWaves;     // a wave's slots
+__global__ __launch_bounds__(kNllNT) void split_nll_kernel(SplitArgs a) {
   __shared__ double s_t[kExp64Table];
-  __shared__ double s_ps[kWpb];
-  const int row = (int)(blockIdx.x / (unsigned)a.ns), sl = (int)(blockIdx.x % (unsigned)a.ns);
+  __shared__ double s_e[kNllSlots][kWave];
+  const int row = (int)(blockIdx.x / kNllParts), part = (int)(blockIdx.x % kNllParts);
   const int tid = (int)threadIdx.x, lane = lane_id(), wv = wave_id();
   const float* x = a.logits + (int64_t)row * a.V;
   const int n = (int)a.V;
   const RowWork w = row_work(a, row);
-  const int i0 = sl * kSplitSlice + wv * kGpw * kGroup + 4 * lane;
-  f32x4 v[kGpw];
-  load_groups(x, i0 - 4 * lane, n, v);
+  const int t = part * kWave + lane;  // the thread of row_nll_kernel
+  const bool vec = n % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+  const int slots = vec ? (n / 4 + kNllThreads - 1) / kNllThreads * 4 : (n + kNllThreads - 1) / kNllThreads;
+  float v[kNllPer];
+  auto first = [&](int s0) { return s0 + wv * kNllPer; };  // this wave's first slot of the chunk
+  // element of slot s (past the row: none)
+  auto elem = [&](int s) { return vec ? 4 * (t + (s >> 2) * kNllThreads) + (s & 3) : t + s * kNllThreads; };
+  auto load = [&](int s0) __attribute__((always_inline)) {
+    if (vec) {
+#pragma unroll
+      for (int k = 0; k < kNllPer; k += 4) {
+        const int i = elem(first(s0) + k);
+        f32x4 q{};
+        if (i < n) q = *reinterpret_cast<const f32x4*>(x + i);
+        v[k] = q.x;
+        v[k + 1] = q.y;
+        v[k + 2] = q.z;
+        v[k + 3] = q.w;
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < kNllPer; ++k) {
+        const int i = elem(first(s0) + k);
+        v[k] = i < n ? x[i] : 0.0f;
+      }
+    }
+  };
+  load(0);
   if (tid < kExp64Table) s_t[tid] = exp64_table_entry(tid);
   float mx = -__builtin_inff(), unused;
   for (int i = lane; i < w.np; i += kWave) mx = __builtin_fmaxf(mx, w.part[i].x);
   mx = wave_max_f(mx, unused);
   __syncthreads();
   double ps = 0.0;
+  for (int s0 = 0; s0 < slots; s0 += kNllSlots) {
 #pragma unroll
-  for (int g = 0; g < kGpw; ++g) {
-    const float l[4] = {v[g].x, v[g].y, v[g].z, v[g].w};
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (i0 + g * kGroup + j < n) ps += exp64((double)(l[j] - mx), s_t);
+    for (int k = 0; k < kNllPer; ++k)
+      // (+0 past the row: no exponential is -0, so the sum keeps its bits)
+      s_e[wv * kNllPer + k][lane] = elem(first(s0) + k) < n ? exp64((double)(v[k] - mx), s_t) : 0.0;
+    if (s0 + kNllSlots < slots) load(s0 + kNllSlots);
+    __syncthreads();
+    if (wv == 0) {
+#pragma unroll 16
+      for (int k = 0; k < kNllSlots; ++k) ps += s_e[k][lane];
+    }
+    __syncthreads();
   }
+  if (wv != 0) return;
   for (int o = kWave / 2; o > 0; o >>= 1) ps += __shfl_xor(ps, o);
-  if (lane == 0) s_ps[wv] = ps;
-  __syncthreads();
-  if (tid == 0) {
-    double t = s_ps[0];
-    for (int k = 1; k < kWpb; ++k) t += s_ps[k];
-    w.maps[sl] = (uint64_t)__double_as_longlong(t);
-  }
+  if (lane == 0) w.maps[part] = (uint64_t)__double_as_longlong(ps);
 }
 
 // ---------------------------------------------------------------- launch C
 
-// The slices' float64 sums in a fixed tree, and the row's term.
+// The waves' sums in row_nll_kernel's order, and the row's term.
 __global__ __launch_bounds__(kWave) void split_nll_sum_kernel(SplitArgs a) {
   const int row = (int)blockIdx.x, lane = lane_id();
   const RowWork w = row_work(a, row);
   const int t = a.targets[row];
-  const float lt = t >= 0 && t < a.V ? a.logits[(int64_t)row * a.V + t] : __builtin_nanf("");
+  const bool in = t >= 0 && t < a.V;
+  const float lt = in ? a.logits[(int64_t)row * a.V + t] : 0.0f;
+  const double p = lane < kNllParts ? __longlong_as_double((long long)w.maps[lane]) : 0.0;
   float mx = -__builtin_inff(), unused;
-  double s = 0.0;
   for (int i = lane; i < w.np; i += kWave) mx = __builtin_fmaxf(mx, w.part[i].x);
-  for (int i = lane; i < a.ns; i += kWave) s += __longlong_as_double((long long)w.maps[i]);
   mx = wave_max_f(mx, unused);
-  for (int o = kWave / 2; o > 0; o >>= 1) s += __shfl_xor(s, o);
-  if (lane == 0) a.logp[row] = -((double)(lt - mx) - log(s));
+  double s = __shfl(p, 0);
+  for (int k = 1; k < kNllParts; ++k) s += __shfl(p, k);
+  if (lane == 0) a.logp[row] = in ? -((double)(lt - mx) - log(s)) : __builtin_nan("");
 }
 
 // The walk: rounds of 1024 groups, one map per thread, 64 groups per wave.  All
@@ -852,10 +894,6 @@ size_t split_workspace(int kind, int64_t rows, int64_t V, int m) {
   // wave's registers up to kSplitMaxSlices; the grid stays below 2^32 threads.
   const int64_t ns = (V + kSplitSlice - 1) / kSplitSlice;
   if (rows <= 0 || V < kSplitMinV || ns > kSplitMaxSlices || rows * ns >= (int64_t{1} << 23)) return 0;
-  // perplexity's one launch is bound by one CU's float64 units per row, so the
-  // split pays until the rows fill the chip by themselves (V = 128256: 1 row 36 -> 10 us,
-  // 160 rows 46 -> 41, 256 rows 55 -> 60; V = 32000: 8 rows 11.6 -> 10.4, 96 rows
-  // 12.1 -> 14.0)
   if (kind == kSplitNll && (V < kSplitMinNllV || rows > kSplitMaxNllRows)) return 0;
   // softmax's fourth launch pays from longer rows on, or from more rows than
   // CUs (the one launch's second round): 8 x 9000 27.4 -> 29.6 us, 160 x 12288 35.5 ->
@@ -868,6 +906,16 @@ size_t split_workspace(int kind, int64_t rows, int64_t V, int m) {
   size_t b = (size_t)rows * sizeof(SplitRowInfo) + (size_t)(rows * ns) * (kSplitGroups * 8 + kWpb * 8);
   if (kind == kSplitTop) b += (size_t)(rows * ns) * kSplitGroups * 4 + (size_t)rows * kSplitList * 8;
   return b;
+}
+
+// Whether a call that brought the bytes above runs split.  perplexity's one
+// launch is bound by one CU's float64 units per row, so its split pays until the
+// rows fill the chip by themselves (64 / 96 / 128 / 160 rows, one launch against
+// split: V = 50000 16.8 / 17.0 / 17.8 / 18.4 us against 13.9 / 18.1 / 22.5 / 25.4; 65536
+// 20.6 / 20.5 / 20.6 / 24.7 against 14.1 / 19.9 / 23.8 / 27.7; 128256 38 / 41 / 43 / 45
+// against 25 / 32 / 39 / 46).
+bool split_pays(int kind, int64_t rows, int64_t V) {
+  return kind != kSplitNll || rows <= (V < 65536 ? 64 : V < 96000 ? 96 : 128);
 }
 
 hipError_t launch_split(int kind, SplitArgs a, int rows, void* work, hipStream_t s) {
@@ -886,7 +934,7 @@ hipError_t launch_split(int kind, SplitArgs a, int rows, void* work, hipStream_t
   const dim3 grid((unsigned)slices), block(kNT);
   if (kind == kSplitNll) {
     hipLaunchKernelGGL(split_max_kernel<kSplitNll>, grid, block, 0, s, a);
-    hipLaunchKernelGGL(split_nll_kernel, grid, block, 0, s, a);
+    hipLaunchKernelGGL(split_nll_kernel, dim3((unsigned)rows * kNllParts), dim3(kNllNT), 0, s, a);
     hipLaunchKernelGGL(split_nll_sum_kernel, dim3(rows), dim3(kWave), 0, s, a);
   } else if (kind == kSplitTop) {
     hipLaunchKernelGGL(split_max_kernel<kSplitTop>, grid, block, 0, s, a);

@@ -177,6 +177,38 @@ def test_nan_rows_as_in_one_launch(pkg, torch, V):
         assert torch.equal(gp.view(torch.int32), pr.view(torch.int32)), (V, n)
 
 
+@pytest.mark.parametrize("V", [40960, 40961, 50000, 50001, 65537, 128256, 131072, 1 << 20])
+def test_row_nll_has_one_sum(pkg, torch, V):
+    """perplexity's term is the same to the bit with and without a workspace,
+    so it does not depend on how many positions are scored together: full and
+    ragged chunks, on 16 bytes and 4 past, every kind of row."""
+    names, x = _rows(V, V + 1)
+    R = len(names)
+    say(f"[rowsplit] row_nll V={V}, {R} rows")
+    big = torch.empty(R * V + 1, device="cuda")
+    t = torch.from_numpy(np.random.default_rng(V).integers(0, V, size=R).astype(np.int32)).cuda()
+    t[1] = -1
+    t[2] = V
+    vp = ctypes.c_void_p
+    for off in (0, 1):
+        d = big[off:off + R * V].view(R, V)
+        d.copy_(torch.from_numpy(x))
+        got = pkg.row_nll_device(d, t)
+        one = torch.empty(R, dtype=torch.float64, device="cuda")
+        pkg.check(pkg.lib().nls_row_nll(vp(d.data_ptr()), R, V, vp(t.data_ptr()), vp(one.data_ptr()), None), "one launch")
+        same = (got.view(torch.int64) == one.view(torch.int64)) | (got.isnan() & one.isnan())
+        assert same.all(), (V, off, [names[i] for i in (~same).nonzero().reshape(-1).tolist()])
+
+
+def test_row_nll_of_any_number_of_rows(pkg, torch):
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(200, 50001, generator=g, device="cuda") * 3
+    t = torch.randint(0, 50001, (200,), generator=g, device="cuda", dtype=torch.int32)
+    want = pkg.row_nll_device(x, t)
+    for k in (1, 7, 160, 161):
+        assert torch.equal(pkg.row_nll_device(x[:k], t[:k]), want[:k]), k
+
+
 def test_split_in_a_graph(pkg, torch):
     """The split calls captured once and replayed on changing logits, with
     eager calls between the replays."""
