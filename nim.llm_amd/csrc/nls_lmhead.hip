@@ -27,6 +27,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <atomic>
 
 #include "nls_internal.h"
 #include "nls_lmhead.h"
@@ -1183,13 +1184,33 @@ hipError_t launch_int(const LmHeadCall& c, hipStream_t s) {
   return launch_int_rows<T>(c, nblk, passes, s);
 }
 
+// Activations of a pass of lm_half_kernel (with its tiles, 100 KB of LDS).
+constexpr int64_t kHalfActBytes = 65536;
+
+// The instance's LDS limit at its largest pass, once per device: the limit
+// belongs to the kernel, so a call that set its own size could lower it under
+// another thread's larger launch.
+template <int T, int P, int NB>
+hipError_t half_lds_limit() {
+  static std::atomic<bool> done[64];
+  int dev = 0;
+  const hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  const bool kept = dev >= 0 && dev < 64;
+  if (kept && done[dev].load(std::memory_order_acquire)) return hipSuccess;
+  const hipError_t e2 = hipFuncSetAttribute(reinterpret_cast<const void*>(lm_half_kernel<T, P, NB>),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize,
+                                            (kLmNT / 64) * half_lds_wave<P>() + (int)kHalfActBytes);
+  if (e2 == hipSuccess && kept) done[dev].store(true, std::memory_order_release);
+  return e2;
+}
+
 template <int T, int P, int NB>
 hipError_t launch_half(const FloatArgs& a, int64_t c8, hipStream_t s) {
   const int64_t per = (kLmNT / 64) * (64 / P);
   const size_t lds = (kLmNT / 64) * half_lds_wave<P>() + (size_t)NB * (size_t)c8 * 4;
   if (lds > 65536) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(lm_half_kernel<T, P, NB>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    const hipError_t e = half_lds_limit<T, P, NB>();
     if (e != hipSuccess) return e;
   }
   hipLaunchKernelGGL((lm_half_kernel<T, P, NB>), dim3((unsigned)((a.rows + per - 1) / per)), dim3(kLmNT), lds, s, a);
@@ -1204,9 +1225,6 @@ hipError_t launch_half_states(const FloatArgs& a, int64_t c8, hipStream_t s) {
     default: return launch_half<T, P, 4>(a, c8, s);
   }
 }
-
-// Activations of a pass of lm_half_kernel (with its tiles, 100 KB of LDS).
-constexpr int64_t kHalfActBytes = 65536;
 
 template <int T>
 hipError_t launch_float(const LmHeadCall& c, hipStream_t s) {

@@ -283,3 +283,39 @@ def test_half_weights_parity(pkg, name):
     for rows, cols, nb in cases:
         print(f"lm_head two-byte {name} rows={rows} cols={cols} nb={nb}", flush=True)
         run_case(pkg, t, rows, cols, nb, seed=rows + cols)
+
+
+@pytest.mark.gpu
+def test_half_weights_from_two_threads(pkg):
+    """Two host threads with two-byte weights of unlike lengths, both past the
+    default LDS size of one kernel instance: no launch is refused for the
+    other's size, and every call gives its own logits."""
+    import threading
+
+    import torch
+
+    cases, errors = [], []
+    for cols, rows in ((5456, 1000), (2900, 40)):
+        g = torch.Generator(device="cuda").manual_seed(cols)
+        w = torch.empty(rows, cols, dtype=torch.float16, device="cuda").normal_(generator=g).view(torch.uint8).reshape(-1)
+        x = torch.randn(3, cols, device="cuda", generator=g)
+        cases.append((w, rows, cols, x, pkg.lm_head(w, 1, rows, cols, x)))
+    torch.cuda.synchronize()
+
+    def run(case):
+        w, rows, cols, x, want = case
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                outs = [pkg.lm_head(w, 1, rows, cols, x) for _ in range(600)]
+                torch.cuda.current_stream().synchronize()
+                assert all(torch.equal(o, want) for o in outs[::50])
+        except Exception as e:  # noqa: BLE001
+            errors.append(repr(e))
+
+    print("lm_head from two threads", flush=True)
+    threads = [threading.Thread(target=run, args=(c,)) for c in cases]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors[:2]
