@@ -142,7 +142,7 @@ __global__ __launch_bounds__(NT) void top_tokens_kernel(const float* __restrict_
     mx = in.mx;
     s = in.sum;
     nl = in.count;
-    t0 = f2key(in.bound);
+    t0 = in.bound;
     if (tid < kExpfPow2Count) s_pow2[tid] = kExpfPow2J64[tid];
     for (int i = tid; i < min(nl, kTopList); i += NT) list[i] = pre_list[(int64_t)row * kTopList + i];
     __syncthreads();

@@ -24,8 +24,8 @@ constexpr float kSplitErr = 0x1p-22f;
 
 struct SplitRowInfo {
   float mx, sum;
-  float bound;  // topTokens: every logit >= bound is listed
-  int count;    // topTokens: listed logits (zeroed by the first launch)
+  uint32_t bound;  // topTokens: every logit whose key reaches it is listed (both
+  int count;       // zeroed by the first launch); the logits listed
   int pad[4];
 };
 

@@ -54,6 +54,8 @@ constexpr int kHeadGroups = 1;                   // the row's first group is add
 constexpr int kWalkNT = 1024;                    // groups per round of the walk, one per thread
 constexpr int kSlots = kWalkNT / kWave - 1;      // crossing groups prepared per round, one per wave
                                                  // (the last wave adds the row's first group)
+constexpr int kManyLanes = 24;                   // topTokens: lanes with a logit to list, of a wave that looks for
+                                                 // a bound of its own
 constexpr float kLog2e = 1.44269502162933349609375f;
 
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
@@ -279,7 +281,10 @@ __global__ __launch_bounds__(kNT) void split_max_kernel(SplitArgs a) {
   const RowWork w = row_work(a, row);
   f32x4 v[kGpw];
   load_groups(x, sl * kSplitSlice + wv * kGpw * kGroup, n, v);
-  if (sl == 0 && tid == 0) w.info->count = 0;
+  if (sl == 0 && tid == 0) {
+    w.info->count = 0;
+    w.info->bound = 0u;
+  }
   float m = -__builtin_inff(), rowm;
 #pragma unroll
   for (int g = 0; g < kGpw; ++g)
@@ -313,7 +318,7 @@ template <int KIND>
 __global__ __launch_bounds__(kNT, 8) void split_terms_kernel(SplitArgs a) {
   __shared__ double s_pow2[kExpfPow2Count];
   const int row = (int)(blockIdx.x / (unsigned)a.ns), sl = (int)(blockIdx.x % (unsigned)a.ns);
-  const int tid = (int)threadIdx.x, lane = lane_id(), wv = wave_id();
+  const int lane = lane_id(), wv = wave_id();
   const float* x = a.logits + (int64_t)row * a.V;
   const int n = (int)a.V;
   const RowWork w = row_work(a, row);
@@ -342,24 +347,77 @@ __global__ __launch_bounds__(kNT, 8) void split_terms_kernel(SplitArgs a) {
   P = wave_sum_f(P);
   if (KIND == kSplitTop) {
     // The list's bound.  The row's 256-element maxima, merged to 64: the m-th
-    // largest of those is a logit that m distinct elements reach.  It is
+    // largest of those is a logit that m distinct elements reach.  Bounds are
     // lowered by more than the spacing at which l - mx, the exponential and
     // the division can round unlike logits to one probability.
     uint32_t key = 0u;
     for (int i = lane; i < a.ns * kSplitGroups; i += kWave) key = max(key, f2key(w.gmax[i]));
-    float th = key2f(wave_kth_largest(key, a.m));
-    th -= 0x1p-18f * __builtin_fmaxf(1.0f, __builtin_fmaxf(__builtin_fabsf(mx), __builtin_fabsf(th)));
-    if (sl == 0 && tid == 0) w.info->bound = th;
+    auto lowered = [&](uint32_t k) {
+      const float t = key2f(k);
+      return t - 0x1p-18f * __builtin_fmaxf(1.0f, __builtin_fmaxf(__builtin_fabsf(mx), __builtin_fabsf(t)));
+    };
+    float th = lowered(wave_kth_largest(key, a.m));
+    if (me == 0 && lane == 0) atomicMax(&w.info->bound, f2key(th));
+    float lm = -__builtin_inff();
 #pragma unroll
-    for (int g = 0; g < kGpw; ++g) {
-      const float l[4] = {v[g].x, v[g].y, v[g].z, v[g].w};
-      const int i0 = (g0 + g) * kGroup + 4 * lane;
+    for (int g = 0; g < kGpw; ++g)
+      lm = __builtin_fmaxf(lm, __builtin_fmaxf(__builtin_fmaxf(v[g].x, v[g].y), __builtin_fmaxf(v[g].z, v[g].w)));
+    const int lanes = (int)__popcll(__ballot(lm >= th));
+    if (lanes > kManyLanes) {  // uniform
+      // A wave that holds many of the row's largest logits side by side (rows that
+      // rise or fall) has bounds of its own: the m-th largest of its lanes' maxima,
+      // and the value that the four neighbours of m / 4 lanes reach.  Without them the
+      // list overflows and the last launch reads the row several times (falling
+      // rows of 128256, n = 20: one row 194 us, 31 here; 256 rows 300, 120; one launch
+      // 131 and 138).
+      float four = -__builtin_inff();
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (l[j] >= th && i0 + j < n) {
-          const int slot = atomicAdd(&w.info->count, 1);
-          if (slot < kSplitList) w.list[slot] = ((uint64_t)f2key(l[j]) << 32) | (uint32_t)(i0 + j);
+      for (int g = 0; g < kGpw; ++g)
+        four = __builtin_fmaxf(four, __builtin_fminf(__builtin_fminf(v[g].x, v[g].y), __builtin_fminf(v[g].z, v[g].w)));
+      const uint32_t own = max(wave_kth_largest(f2key(lm), a.m), wave_kth_largest(f2key(four), (a.m + 3) / 4));
+      const float tw = lowered(own);
+      if (tw > th) {
+        th = tw;
+        if (lane == 0) atomicMax(&w.info->bound, f2key(th));
+      }
+      int total = 0;
+#pragma unroll
+      for (int g = 0; g < kGpw; ++g) {
+        const float l[4] = {v[g].x, v[g].y, v[g].z, v[g].w};
+        const int i0 = (g0 + g) * kGroup + 4 * lane;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) total += (int)__popcll(__ballot(l[j] >= th && i0 + j < n));
+      }
+      int base = 0;
+      if (lane == 0) base = atomicAdd(&w.info->count, total);
+      base = __builtin_amdgcn_readfirstlane(base);
+      if (base < kSplitList) {
+#pragma unroll
+        for (int g = 0; g < kGpw; ++g) {
+          const float l[4] = {v[g].x, v[g].y, v[g].z, v[g].w};
+          const int i0 = (g0 + g) * kGroup + 4 * lane;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const bool in = l[j] >= th && i0 + j < n;
+            const uint64_t at = __ballot(in);
+            const int slot = base + (int)__popcll(at & lanes_below());
+            if (in && slot < kSplitList) w.list[slot] = ((uint64_t)f2key(l[j]) << 32) | (uint32_t)(i0 + j);
+            base += (int)__popcll(at);
+          }
         }
+      }
+    } else if (lanes > 0) {
+#pragma unroll
+      for (int g = 0; g < kGpw; ++g) {
+        const float l[4] = {v[g].x, v[g].y, v[g].z, v[g].w};
+        const int i0 = (g0 + g) * kGroup + 4 * lane;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (l[j] >= th && i0 + j < n) {
+            const int slot = atomicAdd(&w.info->count, 1);
+            if (slot < kSplitList) w.list[slot] = ((uint64_t)f2key(l[j]) << 32) | (uint32_t)(i0 + j);
+          }
+      }
     }
   }
 

@@ -177,6 +177,41 @@ def test_nan_rows_as_in_one_launch(pkg, torch, V):
         assert torch.equal(gp.view(torch.int32), pr.view(torch.int32)), (V, n)
 
 
+@pytest.mark.parametrize("V", [8192, 50001, 128256])
+def test_top_tokens_list_of_rows_in_order(pkg, torch, V):
+    """Rows whose largest logits lie side by side (rising, falling, in blocks)
+    list few logits for topTokens' last launch, not thousands that would
+    overflow the list; ids and probabilities against the oracle."""
+    i = np.arange(V)
+    rng = np.random.default_rng(V)
+    n = rng.standard_normal(V)
+    x = np.stack([-i * (20.0 / V), i * (20.0 / V), -np.abs(i - V // 2) * (20.0 / V), np.sort(n), -np.sort(n),
+                  np.where((i > 3000) & (i < 4400), 9.0 + n / 8, n)]).astype(np.float32)
+    R = len(x)
+    say(f"[rowsplit] rows in order V={V}")
+    d = torch.from_numpy(x).cuda()
+    vp = ctypes.c_void_p
+    L = pkg.lib()
+    for m in (1, 5, 20, 32, 64):
+        if m > V // 256:
+            continue
+        need = L.nls_rows_workspace(2, R, V, m)
+        work = torch.zeros(need, dtype=torch.uint8, device="cuda")
+        ids = torch.empty(R, m, dtype=torch.int32, device="cuda")
+        pr = torch.empty(R, m, device="cuda")
+        pkg.check(L.nls_top_tokens_ws(vp(d.data_ptr()), R, V, m, vp(ids.data_ptr()), vp(pr.data_ptr()),
+                                      vp(work.data_ptr()), need, None), "nls_top_tokens_ws")
+        torch.cuda.synchronize()
+        # a row's record: two floats, the list's bound and its count, in 32 bytes
+        count = work[:R * 32].view(torch.int32).view(R, 8)[:, 3].cpu().numpy()
+        assert (count >= m).all() and (count <= (1024 if m <= 32 else 2048)).all(), (V, m, count)
+        for r in range(R):
+            want = O.softmax(x[r])
+            order = np.argsort(-want, kind="stable")[:m]
+            assert np.array_equal(ids[r].cpu().numpy(), order), (V, m, r)
+            assert np.array_equal(pr[r].cpu().numpy(), want[order]), (V, m, r)
+
+
 @pytest.mark.parametrize("V", [40960, 40961, 50000, 50001, 65537, 128256, 131072, 1 << 20])
 def test_row_nll_has_one_sum(pkg, torch, V):
     """perplexity's term is the same to the bit with and without a workspace,
