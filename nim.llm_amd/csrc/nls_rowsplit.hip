@@ -927,7 +927,11 @@ __global__ __launch_bounds__(kNT, 8) void split_out_kernel(SplitArgs a) {
     for (int j = 0; j < 4; ++j) {
       bool ok;
       r[j] = (float)((double)expf_cr_quick(d[j], s_pow2, ok) * inv);
-      all = all && ok && r[j] >= 0x1p-126f;
+      // (masked logits: their exponential is 0 from -104 on, with no exact path to take;
+      // 256 x 128256 with 1 logit of 97 unmasked 174 us without this, 145 with it)
+      const bool zero = d[j] <= -104.0f && s == s;
+      r[j] = zero ? 0.0f : r[j];
+      all = all && (zero || (ok && r[j] >= 0x1p-126f));
     }
     if (!all) {
       float e[4];

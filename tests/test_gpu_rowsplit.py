@@ -177,6 +177,30 @@ def test_nan_rows_as_in_one_launch(pkg, torch, V):
         assert torch.equal(gp.view(torch.int32), pr.view(torch.int32)), (V, n)
 
 
+@pytest.mark.parametrize("V", [14337, 50001])
+def test_softmax_of_masked_and_vanishing_terms(pkg, torch, V):
+    """Terms around e^-104 (the last nonzero float32 exponential), subnormal
+    quotients and masked logits (-inf, the lowest float), in runs and
+    scattered: softmax against the oracle, bit for bit."""
+    rng = np.random.default_rng(V)
+    base = rng.standard_normal(V) * 2
+    edge = rng.uniform(-104.5, -103.5, size=V)
+    edge[::7] = -104.0
+    edge[1::7] = np.nextafter(np.float32(-104), np.float32(0))
+    rows = [np.where(rng.random(V) < 0.99, -np.inf, base), np.where(rng.random(V) < 0.99, -3.4028234663852886e38, base),
+            np.where(np.arange(V) % 512 < 256, -np.inf, base), edge, rng.uniform(-106.0, -80.0, size=V),
+            np.where(rng.random(V) < 0.5, edge, -np.inf), rng.uniform(-90.0, -86.0, size=V)]
+    x = np.stack(rows).astype(np.float32)
+    x[3:, 5] = 0.0
+    x[4:, 11] = 0.5
+    say(f"[rowsplit] masked V={V}")
+    got = pkg.softmax_device(torch.from_numpy(x).cuda()).cpu().numpy()
+    for r in range(len(x)):
+        want = O.softmax(x[r])
+        bad = np.flatnonzero(got[r].view(np.uint32) != want.view(np.uint32))
+        assert bad.size == 0, (V, r, bad[:4], got[r][bad[:4]], want[bad[:4]], x[r][bad[:4]])
+
+
 @pytest.mark.parametrize("V", [8192, 50001, 128256])
 def test_top_tokens_list_of_rows_in_order(pkg, torch, V):
     """Rows whose largest logits lie side by side (rising, falling, in blocks)
