@@ -299,6 +299,18 @@ def test_split_in_a_graph(pkg, torch):
             assert torch.equal(a, b), k
 
 
+def test_short_rows_ask_for_no_workspace(pkg):
+    """The lengths below which the Python entry points don't ask for a
+    workspace are the library's: none wanted there, one wanted from there on."""
+    L = pkg.lib()
+    for op, start in pkg._ROWS_WORK_FROM.items():
+        rows = 300 if op == pkg._ROWS_SOFTMAX else 4  # (softmax of few rows splits from 12288 on)
+        assert L.nls_rows_workspace(op, rows, start, 1) > 0, op
+        for r in (1, 4, 160, 300, 5000):
+            assert not any(L.nls_rows_workspace(op, r, v, 1) for v in range(1, start, 127)), (op, r)
+            assert L.nls_rows_workspace(op, r, start - 1, 1) == 0, (op, r)
+
+
 def test_workspace_rule(pkg):
     """A short, odd or missing workspace runs the one-launch kernels; the
     sizes the split covers ask for one."""
