@@ -438,14 +438,20 @@ _ROWS_WORK_FROM = {_ROWS_SOFTMAX: 8192, _ROWS_LOG_PROB: 8192, _ROWS_TOP_TOKENS: 
 
 
 def _rows_work(op: int, x, rows: int, V: int, n: int = 0):
-    """The workspace of a call over the rows of x (None where it wants none),
-    from torch's allocator on the current stream, and its bytes."""
+    """The workspace of a call over the rows of x (None where it wants none, or
+    where the memory has no room for it: topTokens' is half the logits' size for
+    short rows), from torch's allocator on the current stream, and its bytes."""
     if V < _ROWS_WORK_FROM[op]:
         return None, 0
     import torch
 
     need = int(lib().nls_rows_workspace(op, rows, V, n))
-    return (torch.empty(need, dtype=torch.uint8, device=x.device) if need else None), need
+    if not need:
+        return None, 0
+    try:
+        return torch.empty(need, dtype=torch.uint8, device=x.device), need
+    except torch.OutOfMemoryError:  # the calls run without one too
+        return None, 0
 
 
 def top_tokens_device(logits, n: int = 5):

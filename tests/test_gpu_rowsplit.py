@@ -299,6 +299,28 @@ def test_split_in_a_graph(pkg, torch):
             assert torch.equal(a, b), k
 
 
+def test_no_room_for_a_workspace(pkg, torch):
+    """A call whose workspace the memory has no room for runs without one, as it
+    did before there was one (the limit is torch's own, set just above what it
+    holds)."""
+    x = torch.randn(4096, 8192, device="cuda")
+    want = pkg.top_tokens_device(x, 5)
+    need = pkg.lib().nls_rows_workspace(2, 4096, 8192, 5)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    room = need // 2
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + room) / total)
+    say(f"[rowsplit] no room: {need} bytes wanted, {room} left")
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(need, dtype=torch.uint8, device="cuda")
+        got = pkg.top_tokens_device(x, 5)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
 def test_short_rows_ask_for_no_workspace(pkg):
     """The lengths below which the Python entry points don't ask for a
     workspace are the library's: none wanted there, one wanted from there on."""
