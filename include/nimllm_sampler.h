@@ -256,6 +256,9 @@ int nls_log_prob_ws(const float* d_logits, int32_t rows, int64_t vocab, const in
 
 /* Correctly rounded exp on fp32 inputs, on the device: d_out[i] = exp(d_in[i]). */
 int nls_expf_device(const float* d_in, float* d_out, int64_t n, void* stream);
+/* The same, and a NaN wherever one of the kernels' shorter forms of it breaks its
+ * bound (a check, no counterpart in the reference). */
+int nls_expf_forms_device(const float* d_in, float* d_out, int64_t n, void* stream);
 
 /* Measurement hook (no counterpart in the reference): when set, the next
  * nls_sample records hipEvent_t `start` immediately before and `stop`

@@ -36,6 +36,7 @@ EXPORTED = (
     "nls_sample_host_noalloc",
     "nls_synchronize", "nls_rng_uniforms", "nls_get_rng_state", "nls_set_rng_state",
     "nls_top_tokens", "nls_row_nll", "nls_softmax_rows", "nls_log_prob", "nls_expf_device",
+    "nls_expf_forms_device",
     "nls_rows_workspace", "nls_top_tokens_ws", "nls_row_nll_ws", "nls_softmax_rows_ws", "nls_log_prob_ws",
     "nls_profile_next",
     "nls_profile_next_generic", "nls_get_plan", "nls_status_string", "nls_last_error",
@@ -141,6 +142,7 @@ def lib():
         L.nls_softmax_rows_ws.argtypes = L.nls_softmax_rows.argtypes[:-1] + ws
         L.nls_log_prob_ws.argtypes = L.nls_log_prob.argtypes[:-1] + ws
         L.nls_expf_device.argtypes = [vp, vp, ctypes.c_int64, vp]
+        L.nls_expf_forms_device.argtypes = L.nls_expf_device.argtypes
         L.nls_profile_next.argtypes = [vp, vp, vp]
         L.nls_profile_next_generic.argtypes = [vp, vp, vp]
         L.nls_get_plan.argtypes = [vp, P(NlsPlan), P(ctypes.c_int32)]

@@ -1477,7 +1477,13 @@ int nls_log_prob(const float* d_logits, int32_t rows, int64_t vocab, const int32
 
 int nls_expf_device(const float* d_in, float* d_out, int64_t n, void* stream) {
   if (n < 0 || (n > 0 && (!d_in || !d_out))) return NLS_ERR_INVALID_ARGUMENT;
-  NLS_HIP(launch_expf(d_in, d_out, n, reinterpret_cast<hipStream_t>(stream)));
+  NLS_HIP(launch_expf(d_in, d_out, n, false, reinterpret_cast<hipStream_t>(stream)));
+  return NLS_OK;
+}
+
+int nls_expf_forms_device(const float* d_in, float* d_out, int64_t n, void* stream) {
+  if (n < 0 || (n > 0 && (!d_in || !d_out))) return NLS_ERR_INVALID_ARGUMENT;
+  NLS_HIP(launch_expf(d_in, d_out, n, true, reinterpret_cast<hipStream_t>(stream)));
   return NLS_OK;
 }
 

@@ -332,7 +332,7 @@ hipError_t launch_generate_step(const int32_t* d_out, int B, int64_t V, const in
                                 int32_t* row_done, int32_t* hist, int64_t* hist_len, int hcap, hipStream_t s);
 hipError_t launch_accept_device(const int32_t* d_ids, int B, int64_t V, int32_t* hist,
                                 int64_t* hist_len, int hcap, hipStream_t s);
-hipError_t launch_expf(const float* x, float* y, int64_t n, hipStream_t s);
+hipError_t launch_expf(const float* x, float* y, int64_t n, bool forms, hipStream_t s);
 // topTokens over `rows` rows of V logits: n results per row (stride n), n <= kTopMaxN or V <= kTopMaxN
 constexpr int kTopThreads = 1024;
 constexpr int kTopMaxN = 2048;   // largest number of results per row (sorted in LDS)

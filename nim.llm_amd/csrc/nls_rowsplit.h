@@ -18,7 +18,7 @@ constexpr int kSplitMaxNllRows = 160;
 constexpr int kSplitList = 2048;                   // topTokens: logits listed per row
 
 // Relative distance of expf_estimate(d) from the correctly rounded e^d, for
-// d in [-87, 0] (nls_expf_device checks it on every input it is given).  Below
+// d in [-87, 0] (nls_expf_forms_device checks it on every input it is given).  Below
 // -87 both are under 2^-125.
 constexpr float kSplitErr = 0x1p-22f;
 

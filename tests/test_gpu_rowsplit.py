@@ -268,6 +268,22 @@ def test_row_nll_of_any_number_of_rows(pkg, torch):
         assert torch.equal(pkg.row_nll_device(x[:k], t[:k]), want[:k]), k
 
 
+def test_every_form_of_the_exponential(pkg, torch):
+    """The quick form (where it holds) and the estimate's bound on every float32
+    from -0 down to -inf, against the exact exponential."""
+    say("[rowsplit] forms of the exponential: 2.1e9 inputs")
+    L = pkg.lib()
+    step = 1 << 28
+    for a in range(0x80000000, 0xFF800001, step):
+        b = min(a + step, 0xFF800001)
+        x = (torch.arange(a - (1 << 32), b - (1 << 32), dtype=torch.int64, device="cuda").to(torch.int32)).view(torch.float32)
+        want = pkg.expf_device(x)
+        got = torch.empty_like(x)
+        vp = ctypes.c_void_p
+        pkg.check(L.nls_expf_forms_device(vp(x.data_ptr()), vp(got.data_ptr()), x.numel(), None), "forms")
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32)), hex(a)
+
+
 def test_split_in_a_graph(pkg, torch):
     """The split calls captured once and replayed on changing logits, with
     eager calls between the replays."""
