@@ -1,7 +1,8 @@
 """Rows split over workgroups (nls_rowsplit.hip): softmaxInPlace, logProb,
 topTokens and perplexity's term at the sizes where the split starts and ends,
 on rows whose running sum is hard to predict or to keep, against the oracle
-and against the one-launch kernels (the same calls without a workspace)."""
+and against the one-launch kernels (the same calls without a workspace); the
+workspace's bounds."""
 import ctypes
 import math
 import sys
@@ -61,6 +62,27 @@ def _rows(V, seed):
     return list(r), np.stack([v.astype(f) for v in r.values()])
 
 
+def _one_launch(pkg, torch, d, targets, ns=(1, 5, 20, 64)):
+    """log_prob, row_nll and top_tokens of d by the calls without a workspace."""
+    R, V = d.shape
+    L = pkg.lib()
+
+    def p(q):
+        return ctypes.c_void_p(q.data_ptr())
+
+    prob, logp = torch.empty(R, device="cuda"), torch.empty(R, dtype=torch.float64, device="cuda")
+    pkg.check(L.nls_log_prob(p(d), R, V, p(targets), p(prob), p(logp), None), "nls_log_prob")
+    nll = torch.empty(R, dtype=torch.float64, device="cuda")
+    pkg.check(L.nls_row_nll(p(d), R, V, p(targets), p(nll), None), "nls_row_nll")
+    tops = {}
+    for n in ns:
+        ids, pr = torch.empty(R, n, dtype=torch.int32, device="cuda"), torch.empty(R, n, device="cuda")
+        pkg.check(L.nls_top_tokens(p(d), R, V, n, p(ids), p(pr), None), "nls_top_tokens")
+        tops[n] = (ids, pr)
+    torch.cuda.synchronize()
+    return prob, logp, nll, tops
+
+
 # below the split, its first size, ragged sizes, whole and nearly whole slices,
 # real vocabularies, the last size of the split and the first past it
 SIZES = [8191, 8192, 8193, 12287, 12288, 12289, 50001, 128256, 151936, 1 << 20, (1 << 20) + 1]
@@ -90,8 +112,11 @@ def test_split_rows(pkg, torch, V):
         tops = {n: [q.cpu().numpy() for q in pkg.top_tokens_device(d, n)] for n in (1, 5, 20, 64)}
         one = torch.empty(R, V, device="cuda")
         pkg.check(pkg.lib().nls_softmax_rows(vp(d.data_ptr()), R, V, vp(one.data_ptr()), None), "one launch")
-        torch.cuda.synchronize()
         one = one.cpu().numpy()
+        # the same calls without a workspace: the one-launch kernels
+        prob1, logp1, nll1, tops1 = (q.cpu().numpy() if torch.is_tensor(q) else
+                                     {n: [w.cpu().numpy() for w in p] for n, p in q.items()}
+                                     for q in _one_launch(pkg, torch, d, dt))
         in_place = pkg.softmax_device(d2, out=d2).cpu().numpy()
         for i, name in enumerate(names):
             want = O.softmax(x[i])
@@ -101,10 +126,12 @@ def test_split_rows(pkg, torch, V):
                 bad = np.flatnonzero(got.view(np.uint32)[~nan] != want.view(np.uint32)[~nan])
                 assert bad.size == 0, (V, off, name, bad[:4], got[~nan][bad[:4]], want[~nan][bad[:4]])
             wp = want[t[i]]
-            assert (prob[i] == wp) or (np.isnan(wp) and np.isnan(prob[i])), (V, off, name, prob[i], wp)
-            if wp > 0:
-                # the device's float64 log: within 1 ulp of the C library's
-                assert abs(logp[i] - math.log(float(wp))) <= 2 * np.spacing(abs(math.log(float(wp)))), (V, off, name)
+            for pr, lp in ((prob, logp), (prob1, logp1)):
+                assert (pr[i] == wp) or (np.isnan(wp) and np.isnan(pr[i])), (V, off, name, pr[i], wp)
+                if wp > 0:
+                    # the device's float64 log: within 1 ulp of the C library's
+                    assert abs(lp[i] - math.log(float(wp))) <= 2 * np.spacing(abs(math.log(float(wp)))), (V, off, name)
+            assert nll[i] == nll1[i] or (np.isnan(nll[i]) and np.isnan(nll1[i])), (V, off, name, nll[i], nll1[i])
             ref = O.row_nll(x[i], int(t[i]))
             if math.isfinite(ref):
                 # (pairwise sums: the oracle's own, in index order, may be V 2^-53 off)
@@ -117,7 +144,7 @@ def test_split_rows(pkg, torch, V):
             if nan.any():
                 continue  # no order among NaN probabilities
             order = np.argsort(-want, kind="stable")
-            for n, (ids, pr) in tops.items():
+            for n, (ids, pr) in [*tops.items(), *tops1.items()]:
                 m = min(n, V)
                 assert np.array_equal(ids[i], order[:m]), (V, off, name, n, ids[i][:8], order[:8])
                 assert np.array_equal(pr[i], want[order[:m]]), (V, off, name, n)
@@ -259,6 +286,25 @@ def test_row_nll_has_one_sum(pkg, torch, V):
         assert same.all(), (V, off, [names[i] for i in (~same).nonzero().reshape(-1).tolist()])
 
 
+def test_row_nll_of_many_long_rows(pkg, torch):
+    """More rows than the split takes, at a real vocabulary: float64 terms
+    against numpy's, within the roundings of a tree over 2^17 terms."""
+    R, V = 170, 128256
+    say(f"[rowsplit] row_nll {R} x {V}")
+    rng = np.random.default_rng(11)
+    x = (rng.standard_normal((R, V), dtype=np.float32) * np.float32(2.5))
+    x[3, ::2] = -np.inf
+    x[4] = 1.5
+    t = rng.integers(0, V, size=R).astype(np.int32)
+    t[3] = 5
+    assert pkg.lib().nls_rows_workspace(3, R, V, 0) == 0
+    got = pkg.row_nll_device(torch.from_numpy(x).cuda(), torch.from_numpy(t)).cpu().numpy()
+    for r in range(R):
+        d = (x[r] - x[r].max()).astype(np.float64)
+        ref = math.log(float(np.exp(d).sum())) - float(d[t[r]])
+        assert abs(got[r] - ref) <= 1e-12 * max(1.0, abs(ref)), (r, got[r], ref)
+
+
 def test_row_nll_of_any_number_of_rows(pkg, torch):
     g = torch.Generator(device="cuda").manual_seed(3)
     x = torch.randn(200, 50001, generator=g, device="cuda") * 3
@@ -349,9 +395,57 @@ def test_short_rows_ask_for_no_workspace(pkg):
             assert L.nls_rows_workspace(op, r, start - 1, 1) == 0, (op, r)
 
 
+@pytest.mark.parametrize("op", ["softmax", "log_prob", "top_tokens", "row_nll"])
+def test_workspace_contract(pkg, torch, op):
+    """A call writes no byte past the workspace it asked for, and none at all
+    into one that is a byte short, off 16 bytes, or missing: the same results
+    either way."""
+    R, V, n = 3, 50001, 7
+    L, vp = pkg.lib(), ctypes.c_void_p
+    g = torch.Generator(device="cuda").manual_seed(2)
+    x = torch.randn(R, V, generator=g, device="cuda") * 3
+    t = torch.tensor([5, V - 1, 77], dtype=torch.int32, device="cuda")
+    code = ["softmax", "log_prob", "top_tokens", "row_nll"].index(op)
+    need = L.nls_rows_workspace(code, R, V, n)
+    assert need > 0
+    say(f"[rowsplit] workspace of {op}: {need} bytes")
+
+    def p(q):
+        return vp(q.data_ptr())
+
+    def call(work, size):
+        if op == "softmax":
+            outs = [torch.zeros(R, V, device="cuda")]
+            rc = L.nls_softmax_rows_ws(p(x), R, V, p(outs[0]), work, size, None)
+        elif op == "log_prob":
+            outs = [torch.zeros(R, device="cuda"), torch.zeros(R, dtype=torch.float64, device="cuda")]
+            rc = L.nls_log_prob_ws(p(x), R, V, p(t), p(outs[0]), p(outs[1]), work, size, None)
+        elif op == "top_tokens":
+            outs = [torch.zeros(R, n, dtype=torch.int32, device="cuda"), torch.zeros(R, n, device="cuda")]
+            rc = L.nls_top_tokens_ws(p(x), R, V, n, p(outs[0]), p(outs[1]), work, size, None)
+        else:
+            outs = [torch.zeros(R, dtype=torch.float64, device="cuda")]
+            rc = L.nls_row_nll_ws(p(x), R, V, p(t), p(outs[0]), work, size, None)
+        assert rc == 0
+        torch.cuda.synchronize()
+        return outs
+
+    guard = 4096
+    buf = torch.full((guard + need + guard,), 0xAB, dtype=torch.uint8, device="cuda")
+    at = buf.data_ptr() + guard
+    want = call(None, 0)
+    for work, size in ((at, need - 1), (at + 8, need), (at, 0), (None, need)):
+        for a, b in zip(call(vp(work) if work else None, size), want):
+            assert torch.equal(a, b), (op, work, size)
+        assert (buf == 0xAB).all(), (op, work, size)
+    for a, b in zip(call(vp(at), need), want):
+        assert torch.equal(a, b), op
+    assert (buf[:guard] == 0xAB).all() and (buf[guard + need:] == 0xAB).all(), op
+    assert (buf[guard:guard + need] != 0xAB).any(), op  # the split ran
+
+
 def test_workspace_rule(pkg):
-    """A short, odd or missing workspace runs the one-launch kernels; the
-    sizes the split covers ask for one."""
+    """The sizes the split covers ask for a workspace, the others for none."""
     L = pkg.lib()
     assert L.nls_rows_workspace(1, 4, 8191, 0) == 0
     assert L.nls_rows_workspace(1, 4, 8192, 0) > 0
