@@ -555,11 +555,13 @@ def bench_lm_head(args):
     achieved = nbytes / (ms * 1e-3) / 1e9
     path = "int8 activations" if O.matmul_uses_act(t, cols, nb, args.lm_exact) else "dequantise + dotF32"
     if path != "int8 activations":
-        kern = "lm_half_kernel" if args.lm_type in ("F16", "BF16") else "lm_float_kernel"
-    elif nb == 1 and (cols // 32 + 63) // 64 <= 4:
+        kern = "lm_half_kernel" if args.lm_type in ("F16", "BF16") and 8 <= cols < 16392 else "lm_float_kernel"
+    elif (nb if nb < 3 else 4) * ((cols // 32 + 63) // 64) <= 4 and nb <= 4:
         kern = "lm_int1_kernel (activations quantised in the kernel)"
+    elif args.lm_type.endswith("_K"):
+        kern = "quant_act_kernel + lm_batch_kernel (few states of long rows: lm_int_kernel)"
     else:
-        kern = "quant_act_kernel + " + ("lm_batch_kernel" if args.lm_type.endswith("_K") else "lm_int_kernel")
+        kern = "quant_act_kernel + lm_int_kernel"
     res = {"metric": f"LM head calls/sec ({rows} x {cols} {args.lm_type}, nb={nb})",
            "value": 1e3 / ms, "unit": "calls/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
            "ms_per_step": ms, "higher_is_better": True, "scaling": "weak", "vs_baseline": None,

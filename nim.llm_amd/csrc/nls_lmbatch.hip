@@ -32,11 +32,14 @@
 // Bound: at few states the weights' HBM traffic and the making of the planes
 // (about 2 VALU instructions per 4 weights and plane for Q4_K, 7 for Q6_K), at
 // many the matrix unit (two planes, 32 cycles per 32 x 32 x 32 step: 57 us of
-// the 195 at 255 states) and the 5 to 7 VALU instructions per term (89 us),
-// which two waves per SIMD overlap only in part.  128256 x 2048, before (one
-// dot-product instruction per four products, weights re-read per four states)
-// and now: Q4_K, 255 states 4009 -> 207 us; Q6_K, 24 states 571 -> 79 us,
-// 5 states 174 -> 79 us; Q6_K 32000 x 4096, 3 states 99 -> 55 us.
+// about 200 at 255 states) and the 5 to 7 VALU instructions per term (89 us),
+// which two waves per SIMD overlap only in part.  A call's time, activations
+// quantised in it, lm_int_kernel (one dot-product instruction per four products,
+// weights re-read per four states) -> here: 128256 x 2048 Q4_K, 255 states
+// 3961 -> 204 us; Q6_K, 24 states 542 -> 74, 5 states 138 -> 72; 32000 x 4096 Q6_K, 3
+// states 73 -> 49; fewer rows than fill the chip gain too: 8000 x 2048 Q4_K, 24 states
+// 125 -> 16, 16000 x 4096 Q4_K, 8 states 107 -> 27, 8000 x 4096 Q6_K, 5 states 84 -> 47.  Few
+// states of long rows do not (int_kernel_wins, nls_lmhead.hip).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

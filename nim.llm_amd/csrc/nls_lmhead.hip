@@ -16,13 +16,15 @@
 //    (quant.nim:362-374);
 //  * an optional LoRA term (:189-200).
 //
-// Integer sums are exact in any grouping, so the int8 path splits a block
-// across 8 lanes (32 weights each) and adds the lanes' partial sums; only the
-// per-block fp32 terms must be added in order, which one lane per row does
-// from LDS after the wave has formed the terms of its rows.  A dotF32 chain is
-// a sequential fp32 sum, so the float path gives each chain its own lane
-// (8 lanes per row) and combines the chains in the reference's order with DPP
-// exchanges (fp32 addition commutes exactly).
+// Integer sums are exact in any grouping, so the int8 path may split a block
+// across 8 lanes (32 weights each; lm_int1_kernel, lm_int_kernel) or make its
+// products on the matrix cores (lm_batch_kernel, nls_lmbatch.hip); only the
+// per-block fp32 terms must be added in order, which one lane per row does.  A
+// dotF32 chain is a sequential fp32 sum, so the float path gives a lane whole
+// chains: one each (8 lanes per row; lm_float_kernel), or two or four of
+// two-byte weights (lm_half_kernel).  The chains are combined in the
+// reference's order by exchanges between the lanes (fp32 addition commutes
+// exactly).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -913,9 +915,9 @@ __global__ __launch_bounds__(kLmNT) void lm_float_kernel(FloatArgs a) {
 // no bank conflicts); the activations stand in LDS in the order they come.
 // Bound: HBM.  lm_float_kernel, whose lanes own one chain each, moves every
 // weight through LDS as a float of its own, in and out, 64 weights of a row at
-// a time.  F16, one state, lm_float_kernel -> here: 128256 x 2048 179 -> 101 us
-// (5.2 TB/s), 32000 x 4096 86 -> 45, 8000 x 1024 17.5 -> 9.0; four states of 128256 x
-// 2048 543 -> 145.  (P = 1, the activations through the scalar cache: 107 us,
+// a time.  F16, one state, lm_float_kernel -> here: 128256 x 2048 161 -> 101 us
+// (5.2 TB/s), 32000 x 4096 85 -> 44, 8000 x 1024 17.3 -> 9.4; four states of 128256 x
+// 2048 544 -> 136.  (P = 1, the activations through the scalar cache: 107 us,
 // and 235 for four states.)
 template <int P>
 constexpr int half_lds_wave() {

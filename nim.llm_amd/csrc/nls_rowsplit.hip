@@ -31,11 +31,11 @@
 // The launches hand over through memory: an arrival count per row with the
 // walk in its last slice (agent-scope fences, or write-through stores and a
 // wait) cost 30 us of 256 x 128256's 95 us in launch B.
-// Measured, one pass, one launch -> split: topTokens, n = 5, 32 x 128256 147 -> 40 us;
-// softmax 256 x 128256 186 -> 158, 1 x 128256 147 -> 30; logProb 201 x 50001 66 -> 44,
-// 1 x 50001 59 -> 25; perplexity's term 8 x 128256 36 -> 12.  Of softmax's 158 us: A 20,
-// B 57 (about 500 vector instructions a wave, 28 us at full issue), C 20 (latency
-// of one wave), D 51 (262 MB at 5.1 TB/s).
+// Measured, one pass, one launch -> split: topTokens, n = 5, 32 x 128256 146 -> 40 us;
+// softmax 256 x 128256 187 -> 152, 1 x 128256 151 -> 27; logProb 201 x 50001 66 -> 44,
+// 1 x 50001 61 -> 27; perplexity's term 8 x 128256 36 -> 12.  Of softmax's 152 us (traced):
+// A 21, B 59 (about 500 vector instructions a wave, 28 us at full issue), C 21
+// (latency of one wave), D 43 (262 MB at 6.1 TB/s).
 #include "nls_device.h"
 #include "nls_exp64.h"
 #include "nls_rowsplit.h"
@@ -451,13 +451,15 @@ __global__ __launch_bounds__(kNT, 8) void split_terms_kernel(SplitArgs a) {
       const float q = y[g][j] * up;
       const float r = __builtin_rintf(q);
       open = __builtin_fmaxf(open, __builtin_fmaf(q, kSplitErr, __builtin_fabsf(q - r)));
-      t += r;  // exact where settled: each r < 2^20
+      t += r;  // exact where settled: each r <= 2^21, four of them below 2^24
     }
     inc[g] = t;
     // (from 2^-80 on, a term whose estimate was flushed is far below u / 2)
     if (__ballot(!(open < 0.5f)) || gsum[g] == 0.0f || E[g] < -80) late |= 1u << g;
   }
-  wave_sum4(inc);  // sums of integers below 2^28, rounded past 2^24: those leave the binade
+  // sums of integers up to 2^29: exact below 2^24, and rounding keeps any other at
+  // 2^24 or more (it is monotone), where the group leaves the binade
+  wave_sum4(inc);
   {
     // lane g stores group g's map
     float t = inc[0];
