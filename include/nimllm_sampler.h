@@ -238,10 +238,10 @@ int nls_log_prob(const float* d_logits, int32_t rows, int64_t vocab, const int32
 
 /* The four calls above with a device workspace: the rows are split over the
  * GPU's workgroups, which pays above all for few rows (topTokens of 32 x 128256:
- * 147 -> 40 us).  nls_rows_workspace gives the bytes a call wants, 0 where
+ * 146 -> 40 us).  nls_rows_workspace gives the bytes a call wants, 0 where
  * the calls above are as good; `n` counts for topTokens only.  With d_work NULL, not
- * 16-byte aligned, or fewer bytes than that, a call runs as the one above.  Same results
- * either way.  The workspace's contents need no preparation and mean nothing
+ * 16-byte aligned, or fewer bytes than that, a call runs as the one above.  Same results,
+ * to the bit, either way.  The workspace's contents need no preparation and mean nothing
  * afterwards; calls that may overlap need one each. */
 enum { NLS_ROWS_SOFTMAX = 0, NLS_ROWS_LOG_PROB = 1, NLS_ROWS_TOP_TOKENS = 2, NLS_ROWS_NLL = 3 };
 size_t nls_rows_workspace(int32_t op, int32_t rows, int64_t vocab, int32_t n);
